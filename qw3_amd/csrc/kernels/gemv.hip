@@ -1,9 +1,11 @@
 // gemv.hip -- fp32 products with quantised weights, C[m][n] = A[m] . W[n].
 //
 // The general-purpose kernel behind the reference's vec_matmul_* and
-// matmul_quantized_batch entry points (src/ds3_metal.h:90-161) and the router
-// logits.  Lanes split K in 32-weight units; a group of G lanes owns one row
-// and decodes each unit once for a tile of up to 8 tokens staged in LDS.
+// matmul_quantized_batch entry points (src/ds3_metal.h:90-161).  Lanes split K
+// in 32-weight units; a group of G lanes owns one row and decodes each unit
+// once for a tile of up to 8 tokens staged in LDS.  It serves one token with
+// few or short rows, F32 rows, and rows that are no multiple of 256; the other
+// quantised products run on k_gemm32.
 //
 // One token over long matrices (the output head, 151,936 x 2048, and the
 // decode projections, src/ds3_engine.c:181-247) goes to k_gemv1 instead: the
@@ -152,6 +154,131 @@ static hipError_t launch_gemv1(int type, const float *x, const uint8_t *w, float
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_gemm32: C[m][n] = A[m] . W[n] for a few rows of A, in fp32 on the matrix
+// cores (v_mfma_f32_16x16x4_f32: fp32 operands, fp32 accumulation).
+// k_gemv decodes every weight again for each group of 8 rows of A and takes
+// one LDS read per multiply; here a weight is decoded once for 16 * MB rows
+// and the products leave the VALU.
+//
+// A workgroup takes 16 rows of W and 16 * MB rows of A; its waves split K in
+// steps of 256 (wave w takes steps w, w + NW, ...), so that the few-row
+// products of an expert (27 x 2048 -> 768 is 48 such tiles) still put 8 waves
+// on every tile.  Lane group g (lanes 16g..16g+15) decodes units g and g + 4
+// of its row per step and reads A at the same K positions, so the MFMA's K
+// order is a permutation shared by both operands.
+//
+// Sums: chains of 8 MFMAs (32 products, as long as k_gemv's lane sums), added
+// as a tree over the unit, the step and, through LDS, the waves.  One chain
+// per wave and step put the error against 64-bit sums at 2.9e-7 (relative
+// L2, K = 2048) where k_gemv has 1.2e-7; this order has 1.2e-7 too.
+//
+// Measured (MI355X, us per call enqueued back to back, k_gemv before): 27 x
+// 2048 -> 768 in Q4_K 73.4 -> 7.6, Q6_K 46.0 -> 8.7, Q8_0 128 -> 8.6; 63 x 2048
+// -> 4096 480 / 259 / 920 -> 22 / 22 / 34; 40 x 4096 -> 8192 1215 / 657 / 2341
+// -> 64 / 66 / 93 (33 TFLOP/s).  Small products are bound by the launch and
+// one memory latency, large ones by the fp32 MFMA rate (33 cycles per
+// 16x16x4).
+// ---------------------------------------------------------------------------
+typedef float g32_f4 __attribute__((ext_vector_type(4)));
+typedef float g32_f4u __attribute__((ext_vector_type(4), aligned(4)));   // rows of A start on any float
+
+constexpr int G32_TILE = 16;
+constexpr int G32_STEP = 256;
+constexpr int G32_MAX_WAVES = 8;
+
+// unit_decode with Q8_0's 34 bytes read as 10 aligned dwords in three loads
+// (any byte alignment) instead of two dwords for each code dword.
+template <int TYPE>
+__device__ __forceinline__ void g32_decode(const uint8_t *row, int u, float (&w)[32], int (&k0)[4])
+{
+    if constexpr (TYPE == T_Q8_0) {
+        typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
+        typedef uint32_t u2 __attribute__((ext_vector_type(2), aligned(4)));
+        const uint8_t *blk = row + (size_t)u * 34;
+        const uint32_t sh = (uint32_t)((uintptr_t)blk & 3);
+        const uint8_t *p = blk - sh;
+        const u4 a = *(const u4 *)p, b = *(const u4 *)(p + 16);
+        const u2 c = *(const u2 *)(p + 32);
+        const uint32_t q[10] = { a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y };
+        const float d = h2f(__builtin_amdgcn_alignbyte(q[1], q[0], sh) & 0xffffu);
+        const bool up = sh >= 2;                     // the codes start at byte sh + 2
+        const uint32_t cs = (sh + 2) & 3;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint32_t v = __builtin_amdgcn_alignbyte(up ? q[i + 2] : q[i + 1], up ? q[i + 1] : q[i], cs);
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[4 * i + j] = (float)(int8_t)byte_of(v, j) * d;
+        }
+#pragma unroll
+        for (int s = 0; s < 4; s++) k0[s] = 32 * u + 8 * s;
+    } else {
+        unit_decode<TYPE>(row, u, w, k0);
+    }
+}
+
+template <int TYPE, int MB>
+__global__ void __launch_bounds__(WAVE * G32_MAX_WAVES)
+k_gemm32(const float *__restrict__ A, int64_t lda, const uint8_t *__restrict__ W, uint64_t stride,
+         float *__restrict__ C, int64_t ldc, int M, int N, int K)
+{
+    __shared__ g32_f4 part[G32_MAX_WAVES][MB][WAVE];
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
+    const int g = lane >> 4, c = lane & 15;
+    const int n = blockIdx.x * G32_TILE + c, m0 = blockIdx.y * G32_TILE * MB;
+    // rows past the end repeat the last one; their results are not stored
+    const uint8_t *row = W + (uint64_t)min(n, N - 1) * stride;
+    const float *a[MB];
+    g32_f4 acc[2][MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) {
+        a[mb] = A + (int64_t)min(m0 + G32_TILE * mb + c, M - 1) * lda;
+        acc[0][mb] = acc[1][mb] = g32_f4{ 0.f, 0.f, 0.f, 0.f };
+    }
+    for (int s = wave; s < K / G32_STEP; s += nw)
+#pragma unroll
+        for (int hv = 0; hv < 2; hv++) {
+            g32_f4 x[MB][8];
+            float w[32];
+            int k0[4];
+            g32_decode<TYPE>(row, 8 * s + g + 4 * hv, w, k0);
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) x[mb][i] = *(const g32_f4u *)(a[mb] + k0[i >> 1] + 4 * (i & 1));
+            // chains of 8 MFMAs (32 products), added as a tree
+            g32_f4 p[4][MB];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++) p[j][mb] = g32_f4{ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int mb = 0; mb < MB; mb++)
+                        p[j][mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[mb][2 * j + (i >> 2)][i & 3], w[8 * j + i],
+                                                                       p[j][mb], 0, 0, 0);
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) acc[hv][mb] += (p[0][mb] + p[1][mb]) + (p[2][mb] + p[3][mb]);
+        }
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) part[wave][mb][lane] = acc[0][mb] + acc[1][mb];
+    __syncthreads();
+    for (int mb = wave; mb < MB; mb += nw) {
+        g32_f4 q[G32_MAX_WAVES];
+#pragma unroll
+        for (int w = 0; w < G32_MAX_WAVES; w++) q[w] = w < nw ? part[w][mb][lane] : g32_f4{ 0.f, 0.f, 0.f, 0.f };
+        const g32_f4 v = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int m = m0 + G32_TILE * mb + 4 * g + i;
+            if (m < M && n < N) C[(int64_t)m * ldc + n] = v[i];
+        }
+    }
+}
+
 constexpr int GEMV_MT = 8;            // tokens per tile
 constexpr int GEMV_TPB = 256;
 
@@ -249,6 +376,40 @@ static hipError_t gemv_type(int G, dim3 grid, size_t lds, hipStream_t s, const f
     return hipGetLastError();
 }
 
+template <int TYPE>
+static hipError_t gemm32_type(const float *A, int64_t lda, const uint8_t *w, uint64_t stride, float *C, int64_t ldc,
+                              int M, int N, int K, hipStream_t s)
+{
+    const int nt = (N + G32_TILE - 1) / G32_TILE, steps = K / G32_STEP;
+    const int nw = steps < G32_MAX_WAVES ? steps : G32_MAX_WAVES;
+    // as many rows of A per workgroup as leave two workgroups per CU
+    int mb = 4;
+    while (mb > 1 && (M <= G32_TILE * mb / 2 || (int64_t)nt * ((M + G32_TILE * mb - 1) / (G32_TILE * mb)) < 512)) mb /= 2;
+    const dim3 grid((unsigned)nt, (unsigned)((M + G32_TILE * mb - 1) / (G32_TILE * mb))), block(WAVE * nw);
+    switch (mb) {
+    case 1: hipLaunchKernelGGL((k_gemm32<TYPE, 1>), grid, block, 0, s, A, lda, w, stride, C, ldc, M, N, K); break;
+    case 2: hipLaunchKernelGGL((k_gemm32<TYPE, 2>), grid, block, 0, s, A, lda, w, stride, C, ldc, M, N, K); break;
+    default: hipLaunchKernelGGL((k_gemm32<TYPE, 4>), grid, block, 0, s, A, lda, w, stride, C, ldc, M, N, K); break;
+    }
+    return hipGetLastError();
+}
+
+// k_gemm32's shapes: quantised rows of whole 256-wide steps.  From two rows of
+// A it always wins (MI355X, k_gemv against k_gemm32, Q4_K / Q6_K / Q8_0: 2 x
+// 2048 -> 768 10.2 / 8.6 / 13.6 against 7.0 / 7.6 / 6.6 us; 63 x 512 -> 300
+// 13.5 / 11.2 / 20.5 against 6.5 / 6.5 / 5.5 us).  One row fills 1/16 of the
+// tile but still decodes faster with every lane group on its own unit: 1024 ->
+// 20,000 26.3 / 18.1 / 44.2 against 11.0 / 12.9 / 10.5 us, 512 -> 131,072 47.5
+// / 39.0 / 77.8 against 29.4 / 35.3 / 30.3, 1024 -> 4096 8.0 / 6.4 / 11.5
+// against 6.5 / 6.4 / 6.4.  One row stays on k_gemv below 2048 rows of W (1024
+// -> 700 5.9 / 5.6 against 6.4 / 6.5 us in Q4_K / Q6_K) and at an odd number
+// of steps (768 -> 32,000 11.2 / 11.1 against 13.8 / 16.2 us).
+static bool gemm32_ok(int type, int M, int N, int K, const float *wnorm2)
+{
+    if (wnorm2 != nullptr || K % G32_STEP != 0 || (type != T_Q4_K && type != T_Q6_K && type != T_Q8_0)) return false;
+    return M >= 2 || (N >= 2048 && K % (2 * G32_STEP) == 0);
+}
+
 // Lanes per row: the largest power of two dividing the unit count (no idle
 // lanes), capped at 64.
 static int lanes_per_row(int units)
@@ -263,6 +424,13 @@ hipError_t launch_gemv(int type, const float *A, int64_t lda, const uint8_t *w, 
 {
     if (!gemv_type_ok(type, K) || M <= 0 || N <= 0) return hipErrorInvalidValue;
     if (gemv1_ok(type, w, stride, M, K, wnorm2)) return launch_gemv1(type, A, w, C, N, K, s);
+    if (gemm32_ok(type, M, N, K, wnorm2)) {
+        switch (type) {
+        case T_Q8_0: return gemm32_type<T_Q8_0>(A, lda, w, stride, C, ldc, M, N, K, s);
+        case T_Q4_K: return gemm32_type<T_Q4_K>(A, lda, w, stride, C, ldc, M, N, K, s);
+        default:     return gemm32_type<T_Q6_K>(A, lda, w, stride, C, ldc, M, N, K, s);
+        }
+    }
     const int G = lanes_per_row(K / 32);
     const int gpw = WAVE / G;
     const int rows_step = (GEMV_TPB / WAVE) * gpw;            // rows one pass of the WG covers

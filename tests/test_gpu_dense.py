@@ -206,3 +206,32 @@ def test_vec_matmul_q4k_half(hip_ready):
     assert hip().ds3_hip_vec_matmul_q4k_half(xb, ds3.Buffer.from_array(raw), yb, K - 32, N, 1152) == -1
     assert hip().ds3_hip_vec_matmul_q4k_half(xb, ds3.Buffer.from_array(raw), yb, K, N, 1000) == -1
     assert hip().ds3_hip_vec_matmul_q4k_half(xb.view(0, K), ds3.Buffer.from_array(raw), yb, K, N, 1152) == -1
+
+
+@pytest.mark.parametrize("t", [12, 14, 8])
+@pytest.mark.parametrize("M,N,K,shift", [(2, 1, 256, 0), (15, 17, 512, 0), (16, 768, 2048, 2), (17, 300, 768, 4),
+                                         (33, 49, 2304, 0), (63, 4112, 1024, 1), (200, 100, 4096, 0), (1, 2049, 512, 2)])
+def test_matmul_quantized_batch_few_rows(hip_ready, t, M, N, K, shift):
+    """Products below the MFMA row count (or of shapes that path does not
+    take) run in fp32 on the matrix cores: partial tiles of rows and columns, 1 to 16 K steps over up to 8 waves, A on a 4-byte boundary,
+    and weights `shift` bytes past a dword.  Each result is a chain of 32
+    products and a tree of at most 12 sums over the exact decoded weights, so
+    it lies within (32 + 12) * 2^-23 of the sum of absolute products (twice
+    the rounding unit, as the matrix core's own rounding is not specified)."""
+    rng = np.random.default_rng(M * 7 + N + K + t)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    raw = normal_matrix(t, 21, N, K)
+    Wf = O.dequantize(t, raw, N * K).reshape(N, K).astype(np.float64)
+    want = A.astype(np.float64) @ Wf.T
+    bound = 44 * 2.0 ** -23 * (np.abs(A).astype(np.float64) @ np.abs(Wf).T)
+    wb = ds3.Buffer.alloc(raw.nbytes + 16)
+    wb.write(raw, offset=shift)
+    ab = ds3.Buffer.alloc(M * K * 4 + 4)
+    ab.write(A, offset=4)
+    cb = ds3.Buffer.alloc(M * N * 4)
+    print(f"  few rows {ds3.TYPE_NAMES[t]} M={M} N={N} K={K} shift={shift}", flush=True)
+    assert hip().ds3_hip_matmul_quantized_batch(ab.view(4, M * K * 4), wb, cb, M, N, K, ds3.row_bytes(t, K), shift,
+                                                t) == 0
+    err = np.abs(cb.read(np.float32, (M, N)).astype(np.float64) - want)
+    print(f"    worst error / bound {float((err / bound).max()):.3f}", flush=True)
+    assert (err <= bound).all()
