@@ -78,6 +78,24 @@ __device__ __forceinline__ void q4k_scale_min(uint32_t s0, uint32_t s1, uint32_t
     mn = (float)b;
 }
 
+// (scale, min) of the two sub-blocks 2(c/2), 2(c/2) + 1 of unit c of a Q4_K
+// block (header words y, z, w), c varying over the lanes: both as byte pairs
+// with per-lane shifts and masks, about 10 instructions; q4k_scale_min with
+// a lane's own j costs about 100 in selects, more than a unit's 64 for its
+// dots.  The masks depend on the lane only and leave the row loops.
+__device__ __forceinline__ void q4k_unit_scales(const uint4 &h, int c, float &sc0, float &mn0, float &sc1, float &mn1)
+{
+    const uint32_t sh = (c & 2) ? 16u : 0u;
+    const bool hi = (c & 4) != 0;
+    const uint32_t ma = hi ? 0xc0c0u : 0x3f3fu, sa = hi ? 2u : 0u, mc = hi ? 0x0f0fu : 0u;
+    const uint32_t a = h.y >> sh, b = h.z >> sh, w = h.w >> sh;
+    const uint32_t sc = ((a & ma) >> sa) | (w & mc), mn = ((b & ma) >> sa) | ((w >> 4) & mc);
+    sc0 = (float)(sc & 0xffu);
+    sc1 = (float)((sc >> 8) & 0xffu);
+    mn0 = (float)(mn & 0xffu);
+    mn1 = (float)((mn >> 8) & 0xffu);
+}
+
 // ---------------------------------------------------------------------------
 // Unit dot products for the fp32 GEMV paths.  x points at the row's K floats
 // (global or LDS).  Q4_K / Q6_K / Q8_0 use sum_i x_i * code_i with the
@@ -115,8 +133,7 @@ __device__ __forceinline__ float unit_dot_q4k(const uint8_t *row, int u, const f
     const uint4 q = *(const uint4 *)(blk + 16 + 16 * c);
     const float d = h2f(hdr.x & 0xffffu), dmin = h2f(hdr.x >> 16);
     float sc0, mn0, sc1, mn1;
-    q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1), sc0, mn0);
-    q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1) + 1, sc1, mn1);
+    q4k_unit_scales(hdr, c, sc0, mn0, sc1, mn1);
     const float *xl = x + 256 * b + 64 * (c >> 1) + 16 * (c & 1);
     const float *xh = xl + 32;
     const uint32_t qw[4] = { q.x, q.y, q.z, q.w };
@@ -211,8 +228,7 @@ __device__ __forceinline__ void unit_decode(const uint8_t *row, int u, float (&w
         const uint4 q = *(const uint4 *)(blk + 16 + 16 * c);
         const float d = h2f(hdr.x & 0xffffu), dmin = h2f(hdr.x >> 16);
         float sc0, mn0, sc1, mn1;
-        q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1), sc0, mn0);
-        q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1) + 1, sc1, mn1);
+        q4k_unit_scales(hdr, c, sc0, mn0, sc1, mn1);
         const float dl = d * sc0, ml = dmin * mn0, dh = d * sc1, mh = dmin * mn1;
         const uint32_t qw[4] = { q.x, q.y, q.z, q.w };
 #pragma unroll

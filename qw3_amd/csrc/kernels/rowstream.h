@@ -110,8 +110,7 @@ __device__ __forceinline__ float g1_unit_dot(const uint8_t *row, int u, const fl
         const uint4 q = *(const uint4 *)(blk + 16 + 16 * c);
         const float d = h2f(hdr.x & 0xffffu), dmin = h2f(hdr.x >> 16);
         float sc0, mn0, sc1, mn1;
-        q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1), sc0, mn0);
-        q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1) + 1, sc1, mn1);
+        q4k_unit_scales(hdr, c, sc0, mn0, sc1, mn1);
         const uint32_t qw[4] = { q.x, q.y, q.z, q.w };
         float dl = 0.f, dh = 0.f;
 #pragma unroll
@@ -146,11 +145,19 @@ __device__ __forceinline__ float g1_unit_dot(const uint8_t *row, int u, const fl
         return d * acc;
     } else {
         static_assert(TYPE == T_Q8_0, "Q4_K, Q6_K or Q8_0");
-        const uint8_t *blk = row + u * 34;
-        const float d = h2f(ld_u16(blk));
+        // rows start on 16 bytes: a block on a dword (even u) or in its middle,
+        // inside 9 dwords either way; one byte permute per code dword
+        const uint32_t sh = 2u * (uint32_t)(u & 1);
+        const uint32_t *p = (const uint32_t *)(row + u * 34 - sh);
+        uint32_t w[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) w[i] = p[i];
+        const float d = h2f((w[0] >> (8 * sh)) & 0xffffu);
+        const uint32_t sel = sh ? 0x07060504u : 0x05040302u;
         float dc = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; i++) dc += dot4(ld_u32_a2(blk + 2 + 4 * i) ^ 0x80808080u, xv + 4 * i);   // int8 + 128
+        for (int i = 0; i < 8; i++)
+            dc += dot4(__builtin_amdgcn_perm(w[i + 1], w[i], sel) ^ 0x80808080u, xv + 4 * i);   // int8 + 128
         return d * (dc - 128.f * ((sx[0] + sx[1]) + (sx[2] + sx[3])));
     }
 }
