@@ -106,7 +106,10 @@ __device__ __forceinline__ void q4k_unit_scales(const uint4 &h, int c, float &sc
 
 __device__ __forceinline__ void cvt4(uint32_t w, float &a, float &b, float &c, float &d)
 {
-    // (float)((w >> 8i) & 0xff) selects v_cvt_f32_ubyte{i}
+    // (float)((w >> 8i) & 0xff) selects v_cvt_f32_ubyte{i}, one instruction per
+    // byte; seeing through a nibble mask on w, the compiler would extract each
+    // byte with a v_bfe_u32 first
+    asm("" : "+v"(w));
     a = (float)(w & 0xffu);
     b = (float)((w >> 8) & 0xffu);
     c = (float)((w >> 16) & 0xffu);
