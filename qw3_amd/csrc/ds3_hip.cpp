@@ -737,31 +737,14 @@ extern "C" int ds3_hip_matmul_quantized_batch(const ds3_hip_buffer_t *A, const d
         return -1;
     }
     if ((int64_t)M >= g.dense_mfma_min && dense_mfma_shape_ok(type, (int)N, (int)K) && M <= 65535) {
-        // fp16 MFMA path: A in fp16, the weights decoded to fp16, fp32
-        // accumulate, on the grouped gate_up kernel as one expert that holds
-        // every row of A (the bucketing lists of M zero expert indices)
-        const int rpi_gu = dense_runs_per_tile((int)N);         // gate_up's run list only: no down
-        const int max_tiles = (int)((M + 63) / 64) + 1;
-        Bump bp;
-        const size_t o_x16 = bp.take((size_t)M * K * 2), o_cnt = bp.take(16), o_off = bp.take(16),
-                     o_ids = bp.take((size_t)M * 4), o_wts = bp.take((size_t)M * 4), o_pos = bp.take((size_t)M * 4),
-                     o_tiles = bp.take((size_t)max_tiles * 4), o_nt = bp.take(16),
-                     o_rg = bp.take((size_t)max_tiles * rpi_gu * 4), o_dg = bp.take((size_t)max_tiles * rpi_gu * 8);
-        uint8_t *ws = ws_get(bp.off);
+        // fp16 MFMA path: A in fp16, the weights decoded to fp16, fp32 accumulate
+        uint8_t *ws = ws_get((size_t)M * K * 2);
         if (!ws) return -1;
-        BucketOut bo{ (int32_t *)(ws + o_cnt), (int32_t *)(ws + o_off), (int32_t *)(ws + o_ids), (float *)(ws + o_wts),
-                      (int32_t *)(ws + o_pos), (int32_t *)(ws + o_tiles), (int32_t *)(ws + o_nt), max_tiles, 64,
-                      (int32_t *)(ws + o_rg), nullptr, (int32_t *)(ws + o_nt) + 1, rpi_gu, 0, (int2 *)(ws + o_dg),
-                      nullptr };
-        hipError_t e = launch_to_f16(fptr(A), (_Float16 *)(ws + o_x16), (int64_t)M * K, g.stream);
-        if (e == hipSuccess) {
-            KScope ks("dense_lists");
-            e = launch_dense_lists((int)M, bo, g.stream);           // one expert holding every row, in order
-        }
+        hipError_t e = launch_to_f16(fptr(A), (_Float16 *)ws, (int64_t)M * K, g.stream);
         if (e == hipSuccess) {
             KScope ks("dense_mfma");
-            e = launch_dense_mfma((const _Float16 *)(ws + o_x16), (int)K, cptr(W) + weight_offset, weight_row_stride,
-                                  type, (int)N, bo, fptr(C), g.stream);
+            e = launch_dense_mfma((const _Float16 *)ws, (int)K, cptr(W) + weight_offset, weight_row_stride, type,
+                                  (int)M, (int)N, fptr(C), g.stream);
         }
         return finish(e, "matmul_quantized_batch");
     }

@@ -185,8 +185,6 @@ hipError_t launch_bucket(const int32_t *idx, const float *scores, int T, int k, 
 // The same lists from launch_route_mark's bitmaps (the rows of these T
 // tokens), one workgroup per 32 tokens.  T <= 2048, k <= 32, E <= 256,
 // max_tiles <= 1280.
-// The lists of a dense product: one expert holding rows 0 .. M-1, in order.
-hipError_t launch_dense_lists(int M, const BucketOut &o, hipStream_t s);
 hipError_t launch_bucket_place(const int32_t *idx, const float *scores, const uint8_t *masks, int T, int k, int E,
                                const BucketOut &o, hipStream_t s);
 
@@ -210,14 +208,11 @@ int device_cu_count();
 void grouped_runs_per_tile(int n_embd, int n_ff, int S, int E, int &rpi_gu, int &rpi_dn);
 
 // Dense C[M][N] = A W^T (fp16 operands, fp32 accumulate) on the grouped
-// gate_up kernel: x16 = A [M][K] in fp16; b = the bucketing lists of one
-// expert holding rows 0 .. M-1 (launch_bucket of M zero indices, k = 1,
-// E = 1, dense_runs_per_tile(N) gate_up runs per token tile); W rows stride
-// bytes apart.  Shapes: dense_mfma_shape_ok.
+// gate_up K loop: x16 = A [M][K] in fp16, W rows stride bytes apart.
+// Shapes: dense_mfma_shape_ok.
 bool dense_mfma_shape_ok(int type, int N, int K);
-int dense_runs_per_tile(int N);
-hipError_t launch_dense_mfma(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int type, int N,
-                             const BucketOut &b, float *c, hipStream_t s);
+hipError_t launch_dense_mfma(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int type, int M, int N,
+                             float *c, hipStream_t s);
 
 // out[t][j] = (accumulate ? out : 0) + sum_k w[t][k] * y[slot_pos[t*k+kk]][j] (+ residual)
 hipError_t launch_combine(const _Float16 *y, const int32_t *slot_pos, const float *wts, int T, int k,

@@ -36,8 +36,6 @@
 #include "common.h"
 #include "launch.h"
 
-#include <type_traits>
-
 namespace ds3k {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -454,8 +452,8 @@ __device__ __forceinline__ void gg_run(const uint8_t *const (&rows)[NB], uint64_
     gg_ring_drain<D, NB>(ring);
 }
 
-// gate_up's K loop: activation rows stream through two LDS chunk buffers of
-// GG_CHUNK_STEPS = 2 K steps each (chunk c of the run = n tile c / (S / 2), K
+// gate_up's K loop (NB = 2; dense products: NB = 1 or 2 sets of weight rows):
+// activation rows stream through two LDS chunk buffers of GG_CHUNK_STEPS = 2 K steps each (chunk c of the run = n tile c / (S / 2), K
 // steps 2 * (c % (S / 2)) .. +1, in buffer c & 1), weights through a ring of
 // D register stages, D - 1 steps ahead.  Issue order, every item
 // unconditional so the wait counts are static:
@@ -464,12 +462,12 @@ __device__ __forceinline__ void gg_run(const uint8_t *const (&rows)[NB], uint64_
 //             wait A(c+1), barrier, then A(c+2) into buffer c & 1
 // a_src(c, dst): this wave's NA DMAs of chunk c (clamped to the run's last
 // chunk) into LDS buffer address dst.
-template <int TYPE, bool AL, int MB, int NA, int D, class ASrc, class Epi>
-__device__ __forceinline__ void gg_run_chunked(const uint8_t *const (&rows)[2], uint64_t tstride, int S, int nnt,
+template <int TYPE, bool AL, int MB, int NA, int D, int NB, class ASrc, class Epi>
+__device__ __forceinline__ void gg_run_chunked(const uint8_t *const (&rows)[NB], uint64_t tstride, int S, int nnt,
                                                uint32_t a_lds, const uint32_t (&lofs)[8], int g, const ASrc &a_src,
                                                const Epi &epi)
 {
-    constexpr int NB = 2, BLK = GgBlk<TYPE>::BLK;
+    constexpr int BLK = GgBlk<TYPE>::BLK;
     using St = GgStage<TYPE, AL>;
     constexpr int NW = NB * St::NLOAD;
     static_assert(NA + (D - 1) * NW <= 63, "vmcnt field holds 0..63");
@@ -484,7 +482,9 @@ __device__ __forceinline__ void gg_run_chunked(const uint8_t *const (&rows)[2], 
 #pragma unroll
         for (int j = 0; j < NB; j++) acc[i][j] = floatx4{ 0.f, 0.f, 0.f, 0.f };
     St ring[D][NB];
-    const uint8_t *wp[NB] = { rows[0], rows[1] };
+    const uint8_t *wp[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) wp[nb] = rows[nb];
     int ls = 0, left = U;
     auto issue = [&](St(&dst)[NB]) {
 #pragma unroll
@@ -654,26 +654,25 @@ struct GgEpiDown {
     }
 };
 
-// Plain-product epilogue (dense C = A W^T on the gate_up kernel): the two
-// row sets of a run are the two halves of W, rows n and n + half; C rows in
-// fp32 (each store instruction writes 4 rows x 16 consecutive columns).
+// Dense epilogue: C rows in fp32, column blocks `second` apart (each store
+// instruction writes 4 rows x 16 consecutive columns).
 struct GgEpiPlain {
     float *c;
-    int N, half, row0, mrows, nt0, wave, lane;
-    template <int MB>
-    __device__ __forceinline__ void store(const floatx4 (&acc)[MB][2], int t) const
+    int64_t ldc, second;
+    int row0, mrows, col0;
+    template <int MB, int NB>
+    __device__ __forceinline__ void store(const floatx4 (&acc)[MB][NB], int) const
     {
-        const int g = lane >> 4, m = lane & 15;
-        const int col = (nt0 + t) * GG_TILE_N + 16 * wave + m;
+        const int lane = threadIdx.x & (WAVE - 1), g = lane >> 4, m = lane & 15;
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int mr = 16 * mb + 4 * g + j;
                 if (mr < mrows) {
-                    float *row = c + (int64_t)(row0 + mr) * N;
-                    row[col] = acc[mb][0][j];
-                    row[half + col] = acc[mb][1][j];
+                    float *p = c + (int64_t)(row0 + mr) * ldc + col0 + m;
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++) p[nb * second] = acc[mb][nb][j];
                 }
             }
     }
@@ -724,9 +723,10 @@ struct GgAChunks {
     }
 };
 
-template <int TYPE, bool AL, int MB, class Epi>
-__device__ __forceinline__ void gg_gate_up_run(const _Float16 *x16, int K, const int32_t *ids, int mrows,
-                                               const uint8_t *const (&rows)[2], uint64_t tstride, int nnt,
+// src_row(r): row r of the run's tile, for r < mrows.
+template <int TYPE, bool AL, int MB, int NB, class SrcRow, class Epi>
+__device__ __forceinline__ void gg_gate_up_run(int K, const SrcRow &src_row, int mrows,
+                                               const uint8_t *const (&rows)[NB], uint64_t tstride, int nnt,
                                                uint32_t a_lds, const uint32_t (&lofs)[8], int wave, int lane,
                                                const Epi &epi)
 {
@@ -739,18 +739,16 @@ __device__ __forceinline__ void gg_gate_up_run(const _Float16 *x16, int K, const
     for (int kk = 0; kk < MB; kk++) {
         const int row = 2 * (wave + GG_WV * kk) + (lane >> 5);
         const int chunk = (lane & 31) ^ (row & 15);
-        as.src[kk] = x16 + (int64_t)ids[row < mrows ? row : 0] * K + 8 * chunk;
+        as.src[kk] = src_row(row < mrows ? row : 0) + 8 * chunk;
     }
     gg_run_chunked<TYPE, AL, MB, GG_CHUNK_STEPS * MB, DS3_GU_DEPTH>(rows, tstride, S, nnt, a_lds, lofs, lane >> 4, as,
                                                                    epi);
 }
 
-// PLAIN: a dense product C[M][2F] = A W^T instead (one expert, W's rows
-// [0, F) in the gate slot and [F, 2F) in the up slot), fp32 C in place of h.
-template <int TYPE, bool PLAIN = false>
+template <int TYPE>
 __global__ void __launch_bounds__(64 * GG_WV)
 k_grouped_gate_up(const _Float16 *__restrict__ x16, int K, ExpertWeights ew, int F, BucketOut b,
-                  _Float16 *__restrict__ h16, int ntb, float *__restrict__ c = nullptr)
+                  _Float16 *__restrict__ h16, int ntb)
 {
     __shared__ __attribute__((aligned(16))) uint8_t smem[GG_GU_LDS];
     const int n_nt = F / GG_TILE_N;
@@ -780,13 +778,11 @@ k_grouped_gate_up(const _Float16 *__restrict__ x16, int K, ExpertWeights ew, int
         const uint8_t *const rows[2] = { wg + r0 * ew.gate_stride, wu + r0 * ew.up_stride };
         const uint64_t tstride = (uint64_t)GG_TILE_N * ew.gate_stride;    // gate and up strides are equal
         const bool al = gg_aligned<TYPE>(wg, wu, ew.gate_stride);
-        using Epi = std::conditional_t<PLAIN, GgEpiPlain, GgEpiGateUp>;
-        Epi epi;
-        if constexpr (PLAIN) epi = GgEpiPlain{ c, 2 * F, F, row0, mrows, nt0, wave, lane };
-        else epi = GgEpiGateUp{ h16, F, row0, mrows, nt0, wave, lane, stage };
-#define DS3_GU_CASE(MBV)                                                                                      \
-    if (al) gg_gate_up_run<TYPE, true, MBV>(x16, K, ids, mrows, rows, tstride, nnt, a_lds, lofs, wave, lane, epi); \
-    else gg_gate_up_run<TYPE, false, MBV>(x16, K, ids, mrows, rows, tstride, nnt, a_lds, lofs, wave, lane, epi);
+        const GgEpiGateUp epi{ h16, F, row0, mrows, nt0, wave, lane, stage };
+        auto src_row = [&](int r) { return x16 + (int64_t)ids[r] * K; };
+#define DS3_GU_CASE(MBV)                                                                                          \
+    if (al) gg_gate_up_run<TYPE, true, MBV>(K, src_row, mrows, rows, tstride, nnt, a_lds, lofs, wave, lane, epi); \
+    else gg_gate_up_run<TYPE, false, MBV>(K, src_row, mrows, rows, tstride, nnt, a_lds, lofs, wave, lane, epi);
         switch (mblocks) {
         case 1: DS3_GU_CASE(1) break;
         case 2: DS3_GU_CASE(2) break;
@@ -841,11 +837,45 @@ k_grouped_down(const _Float16 *__restrict__ h16, int F, ExpertWeights ew, int N,
     }
 }
 
-// Dense C[M][N] = A[M][K] W[N][K]^T on the gate_up kernel: the bucketing
-// lists of one expert holding every row of A (b), x16 = A in fp16.
-template <int TV>
-static hipError_t dense_t(const _Float16 *x16, int K, const ExpertWeights &ew, int N, const BucketOut &b, float *c,
-                          hipStream_t s);
+// Dense C[M][N] = A[M][K] W[N][K]^T: a workgroup takes 64 rows of A and NB
+// sets of 128 rows of W (sets N / NB apart) on gate_up's K loop; its tile comes
+// from the block index, so no list launch precedes it.  Tiles of one W set are
+// consecutive on one XCD, so its weights come through one L2.  Bound by the
+// weight decode, repeated for every 64 rows of A: 512 x 2048 -> 4096 in Q4_K
+// 31.3 -> 21.8 us with the conversion of A (393 TFLOP/s; before, 256-row tiles
+// from a one-workgroup list kernel left half the CUs idle).
+template <int TYPE, int NB>
+__global__ void __launch_bounds__(64 * GG_WV)
+k_dense(const _Float16 *__restrict__ x16, int K, const uint8_t *__restrict__ w, uint64_t stride, int M, int N,
+        int m_tiles, float *__restrict__ c)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * GG_CHUNK];
+    const int idx = gg_list_index(0), nt = idx / m_tiles;
+    if (nt >= N / (NB * GG_TILE_N)) return;              // uniform: the grid is rounded up to the XCDs
+    const int row0 = (idx - nt * m_tiles) * GG_TILE_M, mrows = min(GG_TILE_M, M - row0);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t a_lds = (uint32_t)(uintptr_t)(DS3_LDS void *)smem;
+    uint32_t lofs[8];
+    gg_lofs<TYPE>(lane, lofs);
+    const int col0 = nt * GG_TILE_N + 16 * wave;
+    const uint8_t *rows[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) rows[nb] = w + ((uint64_t)(col0 + (lane & 15)) + (uint64_t)nb * (N / NB)) * stride;
+    const bool al = gg_aligned<TYPE>(w, w, stride);
+    const GgEpiPlain epi{ c, N, N / NB, row0, mrows, col0 };
+    auto src_row = [&](int r) { return x16 + (int64_t)(row0 + r) * K; };
+    const uint8_t *const (&cr)[NB] = rows;
+#define DS3_DENSE_CASE(MBV)                                                                             \
+    if (al) gg_gate_up_run<TYPE, true, MBV>(K, src_row, mrows, cr, 0, 1, a_lds, lofs, wave, lane, epi); \
+    else gg_gate_up_run<TYPE, false, MBV>(K, src_row, mrows, cr, 0, 1, a_lds, lofs, wave, lane, epi);
+    switch ((mrows + 15) / 16) {
+    case 1: DS3_DENSE_CASE(1) break;
+    case 2: DS3_DENSE_CASE(2) break;
+    case 3: DS3_DENSE_CASE(3) break;
+    default: DS3_DENSE_CASE(4) break;
+    }
+#undef DS3_DENSE_CASE
+}
 
 bool grouped_type_ok(int type, int K)
 {
@@ -936,14 +966,28 @@ hipError_t launch_grouped_gate_up(const _Float16 *x16, int K, const ExpertWeight
 }
 
 template <int TV>
-static hipError_t dense_t(const _Float16 *x16, int K, const ExpertWeights &ew, int N, const BucketOut &b, float *c,
+static hipError_t dense_t(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int M, int N, float *c,
                           hipStream_t s)
 {
-    // one n tile per run: a dense product has few token tiles, so the runs,
-    // not the tiles, must fill the CUs
-    const unsigned grid = gg_grid(b.max_tiles * b.rpi_gu);
-    hipLaunchKernelGGL((k_grouped_gate_up<TV, true>), dim3(grid), dim3(64 * GG_WV), 0, s, x16, K, ew, N / 2, b,
-                       nullptr, 1, c);
+    const int64_t m_tiles = (M + GG_TILE_M - 1) / GG_TILE_M, t2 = m_tiles * (N / (2 * GG_TILE_N));
+    const int64_t n_cu = device_cu_count();
+    // 128-row tiles take 2/3 of a 256-row tile's time (A's loads and the loop
+    // are shared by half the weights), so they win when they need at most 3/2
+    // of its rounds of the CUs.  MI355X, us per call with 256- / 128-row tiles,
+    // Q4_K | Q6_K | Q8_0: 64 x 2048 -> 4096 (1 round / 1) 25.5 / 17.0 | 37.1 /
+    // 21.4 | 37.7 / 21.2; 512 x 2048 -> 4096 (1 / 1) 29.3 / 21.6 | 41.0 / 26.0 |
+    // 41.8 / 26.1; 576 x 2048 -> 4096 (1 / 2) 29.7 / 34.6 | 41.5 / 43.0 | 42.3 /
+    // 41.9; 600 x 2048 -> 8192 (2 / 3) 52.2 / 48.6 | 75.0 / 61.4 | 76.3 / 60.7;
+    // 1024 x 2048 -> 8192 (2 / 4) 58.3 / 68.0 | 79.8 / 84.5 | 81.6 / 84.3.
+    const bool one = 2 * ((2 * t2 + n_cu - 1) / n_cu) <= 3 * ((t2 + n_cu - 1) / n_cu);
+    const int64_t grid = ((one ? 2 * t2 : t2) + N_XCD - 1) / N_XCD * N_XCD;
+    if (grid > INT32_MAX / 2) return hipErrorInvalidValue;
+    if (one)
+        hipLaunchKernelGGL((k_dense<TV, 1>), dim3((unsigned)grid), dim3(64 * GG_WV), 0, s, x16, K, w, stride, M, N,
+                           (int)m_tiles, c);
+    else
+        hipLaunchKernelGGL((k_dense<TV, 2>), dim3((unsigned)grid), dim3(64 * GG_WV), 0, s, x16, K, w, stride, M, N,
+                           (int)m_tiles, c);
     return hipGetLastError();
 }
 
@@ -952,28 +996,15 @@ bool dense_mfma_shape_ok(int type, int N, int K)
     return grouped_type_ok(type, K) && K % (256 * DS3_GU_DEPTH) == 0 && N > 0 && N % (2 * GG_TILE_N) == 0;
 }
 
-int dense_runs_per_tile(int N) { return N / 2 / GG_TILE_N; }
-
-hipError_t launch_dense_mfma(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int type, int N,
-                             const BucketOut &b, float *c, hipStream_t s)
+hipError_t launch_dense_mfma(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int type, int M, int N,
+                             float *c, hipStream_t s)
 {
-    const int rg = dense_runs_per_tile(N);
     const uint64_t row_b = type == T_Q8_0 ? (uint64_t)(K / 32) * 34 : (uint64_t)(K / 256) * (type == T_Q4_K ? 144 : 210);
-    if (!dense_mfma_shape_ok(type, N, K) || b.tile_m != GG_TILE_M || b.runs_gu == nullptr || b.desc_gu == nullptr ||
-        b.rpi_gu != rg || b.max_tiles < 1 ||
-        stride < row_b)
-        return hipErrorInvalidValue;
-    ExpertWeights ew{};
-    ew.gate = w;
-    ew.up = w + (uint64_t)(N / 2) * stride;
-    ew.down = nullptr;
-    ew.gate_stride = ew.up_stride = stride;
-    ew.gate_type = ew.up_type = type;
-    ew.table = nullptr;
+    if (!dense_mfma_shape_ok(type, N, K) || M < 1 || stride < row_b) return hipErrorInvalidValue;
     switch (type) {
-    case T_Q4_K: return dense_t<T_Q4_K>(x16, K, ew, N, b, c, s);
-    case T_Q6_K: return dense_t<T_Q6_K>(x16, K, ew, N, b, c, s);
-    case T_Q8_0: return dense_t<T_Q8_0>(x16, K, ew, N, b, c, s);
+    case T_Q4_K: return dense_t<T_Q4_K>(x16, K, w, stride, M, N, c, s);
+    case T_Q6_K: return dense_t<T_Q6_K>(x16, K, w, stride, M, N, c, s);
+    case T_Q8_0: return dense_t<T_Q8_0>(x16, K, w, stride, M, N, c, s);
     default: return hipErrorInvalidValue;
     }
 }

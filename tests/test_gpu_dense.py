@@ -65,6 +65,36 @@ def test_matmul_quantized_batch_mfma(hip_ready, t, M, N, K):
     assert ma <= MFMA_MAX_ABS_UNIT_RMS
 
 
+@pytest.mark.parametrize("t", [12, 14, 8])
+@pytest.mark.parametrize("M,N,K,off", [(65, 256, 512, 0), (16, 1024, 1024, 6), (709, 3328, 512, 0), (709, 3328, 512, 2),
+                                       (64, 66048, 512, 0)])
+def test_matmul_quantized_batch_mfma_tiles(hip_ready, t, M, N, K, off):
+    """Both tile widths of the matrix-core product (128 columns while the wide
+    tiles leave the last round of CUs short, 256 for 709 x 3328), one row in the
+    last token tile, a grid rounded up to the XCDs, rows off 16 bytes, and more
+    than 65,536 columns; the bars of test_matmul_quantized_batch_mfma."""
+    A = np.random.default_rng(M + N + t).standard_normal((M, K)).astype(np.float32)
+    raw = normal_matrix(t, 7, N, K)
+    want = A @ O.dequantize(t, raw, N * K).reshape(N, K).T
+    wb = ds3.Buffer.alloc(raw.nbytes + off)
+    wb.write(raw, offset=off)
+    cb = ds3.Buffer.alloc(M * N * 4)
+    print(f"  dense tiles {ds3.TYPE_NAMES[t]} M={M} N={N} K={K} offset {off}", flush=True)
+    prev = hip().ds3_hip_set_dense_mfma_min_rows(16)
+    try:
+        assert hip().ds3_hip_matmul_quantized_batch(ds3.Buffer.from_array(A), wb, cb, M, N, K, ds3.row_bytes(t, K),
+                                                    off, t) == 0
+    finally:
+        hip().ds3_hip_set_dense_mfma_min_rows(prev)
+    got = cb.read(np.float32, (M, N))
+    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    assert O.rel_l2(got, want) <= MFMA_REL_L2
+    # rounding of A and W to fp16: at most 4e-4 rms relative to the unit-rms output
+    # (2^-11 / sqrt(3) each, times sqrt 2); 4.3 million outputs of one case
+    # reach 6 sigma
+    assert float(np.abs(got - want).max()) / rms <= 6 * 4e-4
+
+
 def test_matmul_quantized_batch_paths(hip_ready):
     """The row count switch: below it the fp32 path (the reference's own
     tolerance), from it the MFMA path; ds3_hip_set_dense_mfma_min_rows moves it."""
