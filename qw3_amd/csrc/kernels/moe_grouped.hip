@@ -453,9 +453,10 @@ __device__ __forceinline__ void gg_run(const uint8_t *const (&rows)[NB], uint64_
 }
 
 // gate_up's K loop (NB = 2; dense products: NB = 1 or 2 sets of weight rows):
-// activation rows stream through two LDS chunk buffers of GG_CHUNK_STEPS = 2 K steps each (chunk c of the run = n tile c / (S / 2), K
-// steps 2 * (c % (S / 2)) .. +1, in buffer c & 1), weights through a ring of
-// D register stages, D - 1 steps ahead.  Issue order, every item
+// activation rows stream through two LDS chunk buffers of GG_CHUNK_STEPS = 2 K
+// steps each (chunk c of the run = n tile c / (S / 2), K steps 2 * (c % (S / 2))
+// .. +1, in buffer c & 1), weights through a ring of D register stages, D - 1
+// steps ahead.  Issue order, every item
 // unconditional so the wait counts are static:
 //   chunk c:  [A(c+1) DMAs]  step 2c: [W(2c+D-1)] wait W(2c) [compute]
 //                            step 2c+1: [W(2c+D)] wait W(2c+1) [compute]
