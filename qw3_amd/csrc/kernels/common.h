@@ -104,23 +104,29 @@ __device__ __forceinline__ void q4k_unit_scales(const uint4 &h, int c, float &sc
 // weight-by-weight dot.
 // ---------------------------------------------------------------------------
 
+// WHOLE: an opaque register copy ahead of the converts.  Seeing through a
+// nibble mask on w, the compiler would extract each byte with a v_bfe_u32
+// first, 40 of the 323 VALU instructions of two Q4_K gate/up rows on the row
+// streams (six layers of eight-stream decode 425 -> 414 us); k_gemm32's decode
+// is 2-6 % faster with it too.  The compiler may then also wait for a unit's
+// loads before it issues the next unit's, so the kernels that read their rows
+// straight from memory choose by shape whether they take it (moe_decode.hip).
+template <bool WHOLE = true>
 __device__ __forceinline__ void cvt4(uint32_t w, float &a, float &b, float &c, float &d)
 {
-    // (float)((w >> 8i) & 0xff) selects v_cvt_f32_ubyte{i}, one instruction per
-    // byte; seeing through a nibble mask on w, the compiler would extract each
-    // byte with a v_bfe_u32 first
-    asm("" : "+v"(w));
+    // (float)((w >> 8i) & 0xff) selects v_cvt_f32_ubyte{i}, one instruction per byte
+    if constexpr (WHOLE) asm("" : "+v"(w));
     a = (float)(w & 0xffu);
     b = (float)((w >> 8) & 0xffu);
     c = (float)((w >> 16) & 0xffu);
     d = (float)(w >> 24);
 }
 
-template <typename XP>
+template <bool WHOLE, typename XP>
 __device__ __forceinline__ float dot4(uint32_t codes, XP x)
 {
     float a, b, c, d;
-    cvt4(codes, a, b, c, d);
+    cvt4<WHOLE>(codes, a, b, c, d);
     return x[0] * a + x[1] * b + x[2] * c + x[3] * d;
 }
 
@@ -128,6 +134,7 @@ template <typename XP>
 __device__ __forceinline__ float sum4(XP x) { return x[0] + x[1] + x[2] + x[3]; }
 
 // Q4_K unit (b, c): returns sum over its 32 weights of w * x.
+template <bool WHOLE>
 __device__ __forceinline__ float unit_dot_q4k(const uint8_t *row, int u, const float *x)
 {
     const int b = u >> 3, c = u & 7;
@@ -143,8 +150,8 @@ __device__ __forceinline__ float unit_dot_q4k(const uint8_t *row, int u, const f
     float dl = 0.f, dh = 0.f, sl = 0.f, sh = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        dl += dot4(qw[i] & 0x0f0f0f0fu, xl + 4 * i);
-        dh += dot4((qw[i] >> 4) & 0x0f0f0f0fu, xh + 4 * i);
+        dl += dot4<WHOLE>(qw[i] & 0x0f0f0f0fu, xl + 4 * i);
+        dh += dot4<WHOLE>((qw[i] >> 4) & 0x0f0f0f0fu, xh + 4 * i);
         sl += sum4(xl + 4 * i);
         sh += sum4(xh + 4 * i);
     }
@@ -152,6 +159,7 @@ __device__ __forceinline__ float unit_dot_q4k(const uint8_t *row, int u, const f
 }
 
 // Q6_K unit (b, h, j).
+template <bool WHOLE>
 __device__ __forceinline__ float unit_dot_q6k(const uint8_t *row, int u, const float *x)
 {
     const int b = u >> 3, h = (u >> 2) & 1, j = u & 3;
@@ -177,7 +185,7 @@ __device__ __forceinline__ float unit_dot_q6k(const uint8_t *row, int u, const f
             const uint32_t nib = (t < 2) ? (ql & 0x0f0f0f0fu) : ((ql >> 4) & 0x0f0f0f0fu);
             const uint32_t two = (hb[w] >> (2 * t)) & 0x03030303u;
             const uint32_t code = nib | (two << 4);          // 0..63 per byte
-            dc += dot4(code, xt + 4 * w);
+            dc += dot4<WHOLE>(code, xt + 4 * w);
             sx += sum4(xt + 4 * w);
         }
         acc += sc * (dc - 32.f * sx);
@@ -186,6 +194,7 @@ __device__ __forceinline__ float unit_dot_q6k(const uint8_t *row, int u, const f
 }
 
 // Q8_0 unit = block u.
+template <bool WHOLE>
 __device__ __forceinline__ float unit_dot_q80(const uint8_t *row, int u, const float *x)
 {
     const uint8_t *blk = row + (size_t)u * 34;
@@ -195,7 +204,7 @@ __device__ __forceinline__ float unit_dot_q80(const uint8_t *row, int u, const f
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const uint32_t q = ld_u32_a2(blk + 2 + 4 * i) ^ 0x80808080u;   // int8 + 128
-        dc += dot4(q, xb + 4 * i);
+        dc += dot4<WHOLE>(q, xb + 4 * i);
         sx += sum4(xb + 4 * i);
     }
     return d * (dc - 128.f * sx);
@@ -211,12 +220,13 @@ __device__ __forceinline__ float unit_dot_f32(const uint8_t *row, int u, const f
     return acc;
 }
 
-template <int TYPE>
+// WHOLE: cvt4's.
+template <int TYPE, bool WHOLE>
 __device__ __forceinline__ float unit_dot(const uint8_t *row, int u, const float *x)
 {
-    if constexpr (TYPE == T_Q4_K) return unit_dot_q4k(row, u, x);
-    else if constexpr (TYPE == T_Q6_K) return unit_dot_q6k(row, u, x);
-    else if constexpr (TYPE == T_Q8_0) return unit_dot_q80(row, u, x);
+    if constexpr (TYPE == T_Q4_K) return unit_dot_q4k<WHOLE>(row, u, x);
+    else if constexpr (TYPE == T_Q6_K) return unit_dot_q6k<WHOLE>(row, u, x);
+    else if constexpr (TYPE == T_Q8_0) return unit_dot_q80<WHOLE>(row, u, x);
     else return unit_dot_f32(row, u, x);
 }
 

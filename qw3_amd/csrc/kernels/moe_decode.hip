@@ -36,6 +36,30 @@ constexpr int N_XCD_DEC = 8;   // MI355X: workgroups go round-robin to 8 XCDs
 #define DS3_SEL_RPW 4          // rows per lane group in the fused-selection gate/up kernel
 #endif
 
+// Where the unit dots take cvt4's opaque copy, for G lanes per row and UPL
+// units per lane.  These kernels live on many loads in flight, which the copy
+// can cost.  Measured both ways on weights that come from memory (MI355X,
+// kernel trace, us without / with):
+//   gate/up, 2-16 tokens: the copy wins with three units per lane (Q4_K 3072 ->
+//     1024, T = 16 126 / 120, Q8_0 321 / 251; Q8_0 1536 -> 768, T = 8 67 / 53; Q6_K
+//     768 -> 512, T = 4 10.7 / 9.7), except Q8_0 at 8 lanes (768 -> 512, T = 2 13.6 /
+//     26.8, T = 16 44 / 70) and Q6_K at more (3072 -> 1024, T = 2 28.3 / 30.0); it
+//     loses with one unit (1024 -> 3072, T = 16 Q4_K 128 / 138, Q8_0 221 / 230) and a
+//     runtime count (1280 -> 3072 Q4_K, T = 4 50 / 55; 1280 -> 1280, T = 8 Q6_K 66 /
+//     72, Q8_0 106 / 111)
+//   gate/up with the selection: it wins for Q8_0 with one unit below 64 lanes
+//     (512 -> 768 12.3 / 11.6, 1024 -> 3072 29.0 / 24.9), else it loses (Q8_0
+//     2048 -> 768 18.2 / 19.3, 1536 -> 768 53 / 69; Q6_K 2048 -> 1024 20.6 / 22.6;
+//     Q4_K 2560 -> 1024 47 / 61)
+//   down: it wins for Q4_K (512 -> 4096, T = 4 25.0 / 22.6) and loses for Q6_K and
+//     Q8_0 (1536 -> 2048, T = 16 102 / 117 and 246 / 255)
+constexpr bool whole_gate_up(int type, int G, int UPL)
+{
+    return UPL == 3 && (type == T_Q4_K || (type == T_Q8_0 && G >= 16) || (type == T_Q6_K && G < 16));
+}
+constexpr bool whole_sel(int type, int G, int UPL) { return type == T_Q8_0 && UPL == 1 && G < 64; }
+constexpr bool whole_down(int type) { return type == T_Q4_K; }
+
 // PAIR: h = swiglu(gate, up).  !PAIR: h = gate projection only, with expert
 // offsets from table column `which` (unfused fallback for mixed types).
 // Lane group (G lanes) per row, UPL = K/32/G units per lane, RPW rows per
@@ -43,7 +67,7 @@ constexpr int N_XCD_DEC = 8;   // MI355X: workgroups go round-robin to 8 XCDs
 // results dropped), so every load of a wave is issued before its first dot
 // product and the wave pays one memory round trip.  Rows of expert e for
 // routed slot `slot` (token row xt), row block rb of the expert.
-template <int GT, int G, int UPL, bool PAIR, int RPW = 2>
+template <int GT, int G, int UPL, bool PAIR, bool WHOLE, int RPW = 2>
 __device__ __forceinline__ void gate_up_rows(const float *__restrict__ xt, int slot, int rb, int e,
                                              const ExpertWeights &ew, int K, int F, int which, float *__restrict__ h)
 {
@@ -64,12 +88,12 @@ __device__ __forceinline__ void gate_up_rows(const float *__restrict__ xt, int s
         const int upl = UPL > 0 ? UPL : K / 32 / G;
 #pragma unroll
         for (int j = 0; j < (UPL > 0 ? UPL : 1); j++) {
-            ag[i] += unit_dot<GT>(grow, gl + G * j, xt);
-            if (PAIR) au[i] += unit_dot<GT>(urow, gl + G * j, xt);
+            ag[i] += unit_dot<GT, WHOLE>(grow, gl + G * j, xt);
+            if (PAIR) au[i] += unit_dot<GT, WHOLE>(urow, gl + G * j, xt);
         }
         for (int j = (UPL > 0 ? UPL : 1); j < upl; j++) {   // shapes without a compile-time count
-            ag[i] += unit_dot<GT>(grow, gl + G * j, xt);
-            if (PAIR) au[i] += unit_dot<GT>(urow, gl + G * j, xt);
+            ag[i] += unit_dot<GT, WHOLE>(grow, gl + G * j, xt);
+            if (PAIR) au[i] += unit_dot<GT, WHOLE>(urow, gl + G * j, xt);
         }
     }
 #pragma unroll
@@ -102,7 +126,7 @@ k_decode_gate_up(const float *__restrict__ x, int64_t ldx, const int32_t *__rest
         return;
     }
     const int r = blockIdx.x - n_exact, slot = r / nx;
-    gate_up_rows<GT, G, UPL, PAIR>(x + (int64_t)(slot / n_used) * ldx, slot, r - slot * nx, idx[slot], ew, K, F,
+    gate_up_rows<GT, G, UPL, PAIR, whole_gate_up(GT, G, UPL)>(x + (int64_t)(slot / n_used) * ldx, slot, r - slot * nx, idx[slot], ew, K, F,
                                    which, h);
 }
 
@@ -360,7 +384,7 @@ k_decode_gate_up_sel(const float *__restrict__ x, int n_used, ExpertWeights ew, 
     const int e = certified ? sel_s[1 + kk]
                             : cert_select_tokens<1>(x, K, cs.w, cs.wstride, cs.ca, ra, t, emit, sel_prod)[kk];
     const uint32_t pf = certified ? prefetch_down_rows(ew, K, n_used, e_rank, lin, nwg) : 0u;
-    gate_up_rows<GT, G, UPL, true, DS3_SEL_RPW>(x + (int64_t)t * K, slot, rb, e, ew, K, F, 0, h);
+    gate_up_rows<GT, G, UPL, true, whole_sel(GT, G, UPL), DS3_SEL_RPW>(x + (int64_t)t * K, slot, rb, e, ew, K, F, 0, h);
     asm volatile("" ::"v"(pf));                // the prefetch loads stay
 }
 
@@ -386,8 +410,8 @@ k_decode_down(const float *__restrict__ h, const int32_t *__restrict__ idx, cons
     const uint8_t *row = wd + (size_t)j * ew.down_stride;
     float acc = 0.f;
 #pragma unroll
-    for (int i = 0; i < (UPL > 0 ? UPL : 1); i++) acc += unit_dot<DT>(row, gl + G * i, hs);
-    for (int i = (UPL > 0 ? UPL : 1); i < F / 32 / G; i++) acc += unit_dot<DT>(row, gl + G * i, hs);
+    for (int i = 0; i < (UPL > 0 ? UPL : 1); i++) acc += unit_dot<DT, whole_down(DT)>(row, gl + G * i, hs);
+    for (int i = (UPL > 0 ? UPL : 1); i < F / 32 / G; i++) acc += unit_dot<DT, whole_down(DT)>(row, gl + G * i, hs);
     acc = group_sum<G>(acc);
     if (gl == 0) part[k * rows_per_wg + grp] = acc;
     __syncthreads();
@@ -453,7 +477,7 @@ __device__ __forceinline__ float unit_dot_q6k_lds(uint32_t row, int u, uint32_t 
             const uint32_t nib = (t < 2) ? (ql & 0x0f0f0f0fu) : ((ql >> 4) & 0x0f0f0f0fu);
             const uint32_t two = (hb[w] >> (2 * t)) & 0x03030303u;
             const uint32_t code = nib | (two << 4);          // 0..63 per byte
-            dc += dot4(code, xt + 4 * w);
+            dc += dot4<false>(code, xt + 4 * w);
             sx += sum4(xt + 4 * w);
         }
         acc += sc * (dc - 32.f * sx);
@@ -478,7 +502,7 @@ __device__ __forceinline__ float unit_dot_q80_lds(uint32_t row, int u, uint32_t 
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const uint32_t q = lds_u32_a2(blk + 2 + 4 * i) ^ 0x80808080u;   // int8 + 128
-        dc += dot4(q, xb + 4 * i);
+        dc += dot4<false>(q, xb + 4 * i);
         sx += sum4(xb + 4 * i);
     }
     return d * (dc - 128.f * sx);

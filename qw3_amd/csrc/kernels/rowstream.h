@@ -115,8 +115,8 @@ __device__ __forceinline__ float g1_unit_dot(const uint8_t *row, int u, const fl
         float dl = 0.f, dh = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            dl += dot4(qw[i] & 0x0f0f0f0fu, xv + 4 * i);
-            dh += dot4((qw[i] >> 4) & 0x0f0f0f0fu, xv + 16 + 4 * i);
+            dl += dot4<true>(qw[i] & 0x0f0f0f0fu, xv + 4 * i);
+            dh += dot4<true>((qw[i] >> 4) & 0x0f0f0f0fu, xv + 16 + 4 * i);
         }
         return (d * sc0) * dl - (dmin * mn0) * (sx[0] + sx[1]) + (d * sc1) * dh - (dmin * mn1) * (sx[2] + sx[3]);
     } else if constexpr (TYPE == T_Q6_K) {
@@ -138,7 +138,7 @@ __device__ __forceinline__ float g1_unit_dot(const uint8_t *row, int u, const fl
             for (int ww = 0; ww < 2; ww++) {
                 const uint32_t ql = (t & 1) ? hig[ww] : low[ww];
                 const uint32_t nib = (t < 2) ? (ql & 0x0f0f0f0fu) : ((ql >> 4) & 0x0f0f0f0fu);
-                dc += dot4(nib | (((hb[ww] >> (2 * t)) & 0x03030303u) << 4), xv + 8 * t + 4 * ww);
+                dc += dot4<true>(nib | (((hb[ww] >> (2 * t)) & 0x03030303u) << 4), xv + 8 * t + 4 * ww);
             }
             acc += sc * (dc - 32.f * sx[t]);
         }
@@ -157,7 +157,7 @@ __device__ __forceinline__ float g1_unit_dot(const uint8_t *row, int u, const fl
         float dc = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++)
-            dc += dot4(__builtin_amdgcn_perm(w[i + 1], w[i], sel) ^ 0x80808080u, xv + 4 * i);   // int8 + 128
+            dc += dot4<true>(__builtin_amdgcn_perm(w[i + 1], w[i], sel) ^ 0x80808080u, xv + 4 * i);   // int8 + 128
         return d * (dc - 128.f * ((sx[0] + sx[1]) + (sx[2] + sx[3])));
     }
 }

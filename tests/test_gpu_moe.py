@@ -662,6 +662,73 @@ def test_decode_down_shapes(hip_ready, n_embd, n_ff, n_expert, n_used):
         assert_close(got, want, rel_l2=5e-5)
 
 
+@pytest.mark.parametrize("gt,dt,n_embd,n_ff", [
+    (8, 8, 512, 768), (8, 8, 768, 512), (8, 8, 1024, 2048), (8, 8, 1536, 1280),      # 16 / 8 / 32 / 16 lanes a row
+    (14, 14, 1024, 1536), (14, 14, 1536, 512),
+    (12, 12, 512, 256), (12, 12, 768, 768), (12, 12, 1024, 1024), (12, 12, 1280, 2048), (12, 12, 3072, 3072),
+])
+def test_decode_row_dots(hip_ready, gt, dt, n_embd, n_ff):
+    """The decode kernels that read their rows straight from memory, with one,
+    three and a runtime number of units per lane and 8 to 64 lanes per row:
+    each choice of the unit dots' code conversion (one token: fused selection;
+    three: separate selection), against the oracle at the decode bar."""
+    spec = W.LayerSpec(gt, gt, dt, 0, W.NORMAL, 0.02, n_embd, n_ff, 16)
+    case = Case(spec, seed=900 + gt + n_embd + n_ff)
+    for T in (1, 3):
+        x = W.fill(W.NORMAL, 8, T, T * n_embd, 0.0, 1.0).reshape(T, n_embd)
+        want, oi, _, probs = case.oracle(x, n_used=4)
+        print(f"  decode rows {ds3.TYPE_NAMES[gt]}/{ds3.TYPE_NAMES[dt]} {n_embd}x{n_ff} T={T}", flush=True)
+        got, gi, _, _ = case.gpu_batch(x, n_used=4)
+        assert index_mismatches(gi, oi, probs) == 0
+        assert_close(got, want, rel_l2=5e-5)
+
+
+def decode_kernel_us(gt, dt, n_embd, n_ff, T, kernel):
+    """Best of five mean durations of one decode kernel over ten layers whose
+    expert blocks (scales and codes at random, results unread) together exceed
+    the caches."""
+    E, k, n_layers = 48, 8, 10
+    rows = ((gt, n_ff, n_embd), (gt, n_ff, n_embd), (dt, n_embd, n_ff))
+    sizes = [E * r * ds3.row_bytes(t, c) for t, r, c in rows]
+    noise = np.random.default_rng(1).integers(0, 256, 1 << 22, dtype=np.uint8)
+
+    def filled(n):
+        b = ds3.Buffer.alloc(n)
+        for o in range(0, n, noise.nbytes):
+            b.write(noise[:min(noise.nbytes, n - o)], offset=o)
+        return b
+
+    layers = [ds3.ExpertTensors(*(filled(n) for n in sizes), gt, gt, dt, n_embd, n_ff) for _ in range(n_layers)]
+    router = ds3.Buffer.from_array(np.random.default_rng(2).standard_normal((E, n_embd)).astype(np.float32))
+    x = ds3.Buffer.from_array(np.random.default_rng(3).standard_normal((T, n_embd)).astype(np.float32))
+    out = ds3.Buffer.alloc(T * n_embd * 4)
+    best = np.inf
+    for rep in range(6):
+        hip().ds3_hip_kernel_timing_reset()
+        hip().ds3_hip_kernel_timing(1)
+        try:
+            for ex in layers:
+                ds3.moe_ffn_batch(x, router, 0, ex, out, T, E, k)
+        finally:
+            hip().ds3_hip_kernel_timing(0)
+        n, ms = ds3.kernel_stats()[kernel]
+        if rep:                                            # the first pass loads the code
+            best = min(best, ms / n * 1e3)
+    return best
+
+
+def test_decode_q8_rows_keep_their_loads_in_flight(hip_ready):
+    """Two tokens' Q8_0 gate/up rows of 768 weights (8 lanes per row, three
+    units per lane) are three quarters of the bytes of rows of 1024 (32 lanes,
+    one unit).  With every unit's loads issued before the first dot they take
+    about 1.3 times as long (13.5 against 10 us); with the units one after
+    another, 2.6 times (27 us)."""
+    a = decode_kernel_us(8, 8, 768, 512, 2, "moe_decode_gate_up")
+    b = decode_kernel_us(8, 8, 1024, 512, 2, "moe_decode_gate_up")
+    print(f"  Q8_0 gate/up, T=2: 768 -> 512 {a:.1f} us, 1024 -> 512 {b:.1f} us", flush=True)
+    assert a < 1.8 * b
+
+
 def test_decode_stack_teacher_forced_config4(hip_ready):
     """Configuration 4 in small: h <- h + MoE_l(h) through distinct layers at
     T = 1 (decode path, residual fused), each layer checked against the
