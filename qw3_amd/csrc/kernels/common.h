@@ -82,7 +82,10 @@ __device__ __forceinline__ void q4k_scale_min(uint32_t s0, uint32_t s1, uint32_t
 // block (header words y, z, w), c varying over the lanes: both as byte pairs
 // with per-lane shifts and masks, about 10 instructions; q4k_scale_min with
 // a lane's own j costs about 100 in selects, more than a unit's 64 for its
-// dots.  The masks depend on the lane only and leave the row loops.
+// dots.  The masks depend on the lane only and leave the row loops.  Kernels
+// bound by their loads and not by these instructions can lose with them all
+// the same, as the compiler then orders the loads differently; they choose by
+// shape (moe_decode.hip).
 __device__ __forceinline__ void q4k_unit_scales(const uint4 &h, int c, float &sc0, float &mn0, float &sc1, float &mn1)
 {
     const uint32_t sh = (c & 2) ? 16u : 0u;
@@ -133,8 +136,9 @@ __device__ __forceinline__ float dot4(uint32_t codes, XP x)
 template <typename XP>
 __device__ __forceinline__ float sum4(XP x) { return x[0] + x[1] + x[2] + x[3]; }
 
-// Q4_K unit (b, c): returns sum over its 32 weights of w * x.
-template <bool WHOLE>
+// Q4_K unit (b, c): returns sum over its 32 weights of w * x.  MASKS: scales
+// by q4k_unit_scales, else by q4k_scale_min.
+template <bool WHOLE, bool MASKS>
 __device__ __forceinline__ float unit_dot_q4k(const uint8_t *row, int u, const float *x)
 {
     const int b = u >> 3, c = u & 7;
@@ -143,7 +147,12 @@ __device__ __forceinline__ float unit_dot_q4k(const uint8_t *row, int u, const f
     const uint4 q = *(const uint4 *)(blk + 16 + 16 * c);
     const float d = h2f(hdr.x & 0xffffu), dmin = h2f(hdr.x >> 16);
     float sc0, mn0, sc1, mn1;
-    q4k_unit_scales(hdr, c, sc0, mn0, sc1, mn1);
+    if constexpr (MASKS) {
+        q4k_unit_scales(hdr, c, sc0, mn0, sc1, mn1);
+    } else {
+        q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1), sc0, mn0);
+        q4k_scale_min(hdr.y, hdr.z, hdr.w, 2 * (c >> 1) + 1, sc1, mn1);
+    }
     const float *xl = x + 256 * b + 64 * (c >> 1) + 16 * (c & 1);
     const float *xh = xl + 32;
     const uint32_t qw[4] = { q.x, q.y, q.z, q.w };
@@ -220,11 +229,11 @@ __device__ __forceinline__ float unit_dot_f32(const uint8_t *row, int u, const f
     return acc;
 }
 
-// WHOLE: cvt4's.
-template <int TYPE, bool WHOLE>
+// WHOLE: cvt4's; MASKS: unit_dot_q4k's.
+template <int TYPE, bool WHOLE, bool MASKS>
 __device__ __forceinline__ float unit_dot(const uint8_t *row, int u, const float *x)
 {
-    if constexpr (TYPE == T_Q4_K) return unit_dot_q4k<WHOLE>(row, u, x);
+    if constexpr (TYPE == T_Q4_K) return unit_dot_q4k<WHOLE, MASKS>(row, u, x);
     else if constexpr (TYPE == T_Q6_K) return unit_dot_q6k<WHOLE>(row, u, x);
     else if constexpr (TYPE == T_Q8_0) return unit_dot_q80<WHOLE>(row, u, x);
     else return unit_dot_f32(row, u, x);

@@ -51,14 +51,27 @@ constexpr int N_XCD_DEC = 8;   // MI355X: workgroups go round-robin to 8 XCDs
 //     (512 -> 768 12.3 / 11.6, 1024 -> 3072 29.0 / 24.9), else it loses (Q8_0
 //     2048 -> 768 18.2 / 19.3, 1536 -> 768 53 / 69; Q6_K 2048 -> 1024 20.6 / 22.6;
 //     Q4_K 2560 -> 1024 47 / 61)
-//   down: it wins for Q4_K (512 -> 4096, T = 4 25.0 / 22.6) and loses for Q6_K and
-//     Q8_0 (1536 -> 2048, T = 16 102 / 117 and 246 / 255)
+//   down: it wins for Q4_K up to 16 lanes (512 -> 4096, T = 4 25.0 / 22.6) and loses
+//     for Q6_K and Q8_0 (1536 -> 2048, T = 16 102 / 117 and 246 / 255)
 constexpr bool whole_gate_up(int type, int G, int UPL)
 {
     return UPL == 3 && (type == T_Q4_K || (type == T_Q8_0 && G >= 16) || (type == T_Q6_K && G < 16));
 }
 constexpr bool whole_sel(int type, int G, int UPL) { return type == T_Q8_0 && UPL == 1 && G < 64; }
-constexpr bool whole_down(int type) { return type == T_Q4_K; }
+constexpr bool whole_down(int type, int G) { return type == T_Q4_K && G <= 16; }
+
+// Where the Q4_K dots take their scales by masks (q4k_unit_scales), else by
+// selects (MI355X, kernel trace, us by selects / by masks):
+//   gate/up, 2-16 tokens: masks with one and three units per lane (1024 -> 3072,
+//     T = 8 71 / 68; 3072 -> 1024, T = 8 102 / 66), selects with a runtime count
+//     (2560 -> 1024, T = 4 41 / 43)
+//   down: masks up to 16 lanes per row (768 -> 2048, T = 8 30.9 / 27.9), selects
+//     above (1024 -> 3072, T = 8 61 / 66; 3072 -> 1024, T = 4 31.5 / 39.7; 6144 -> 512, T = 8
+//     61 / 92)
+// The fused selection's rows take masks throughout (768 -> 512 27.9 / 22.2, 4096 ->
+// 512 26.9 / 25.7, 1280 -> 3072 38.8 / 41.2).
+constexpr bool masks_gate_up(int UPL) { return UPL > 0; }
+constexpr bool masks_down(int G) { return G <= 16; }
 
 // PAIR: h = swiglu(gate, up).  !PAIR: h = gate projection only, with expert
 // offsets from table column `which` (unfused fallback for mixed types).
@@ -67,7 +80,7 @@ constexpr bool whole_down(int type) { return type == T_Q4_K; }
 // results dropped), so every load of a wave is issued before its first dot
 // product and the wave pays one memory round trip.  Rows of expert e for
 // routed slot `slot` (token row xt), row block rb of the expert.
-template <int GT, int G, int UPL, bool PAIR, bool WHOLE, int RPW = 2>
+template <int GT, int G, int UPL, bool PAIR, bool WHOLE, bool MASKS, int RPW = 2>
 __device__ __forceinline__ void gate_up_rows(const float *__restrict__ xt, int slot, int rb, int e,
                                              const ExpertWeights &ew, int K, int F, int which, float *__restrict__ h)
 {
@@ -88,12 +101,12 @@ __device__ __forceinline__ void gate_up_rows(const float *__restrict__ xt, int s
         const int upl = UPL > 0 ? UPL : K / 32 / G;
 #pragma unroll
         for (int j = 0; j < (UPL > 0 ? UPL : 1); j++) {
-            ag[i] += unit_dot<GT, WHOLE>(grow, gl + G * j, xt);
-            if (PAIR) au[i] += unit_dot<GT, WHOLE>(urow, gl + G * j, xt);
+            ag[i] += unit_dot<GT, WHOLE, MASKS>(grow, gl + G * j, xt);
+            if (PAIR) au[i] += unit_dot<GT, WHOLE, MASKS>(urow, gl + G * j, xt);
         }
         for (int j = (UPL > 0 ? UPL : 1); j < upl; j++) {   // shapes without a compile-time count
-            ag[i] += unit_dot<GT, WHOLE>(grow, gl + G * j, xt);
-            if (PAIR) au[i] += unit_dot<GT, WHOLE>(urow, gl + G * j, xt);
+            ag[i] += unit_dot<GT, WHOLE, MASKS>(grow, gl + G * j, xt);
+            if (PAIR) au[i] += unit_dot<GT, WHOLE, MASKS>(urow, gl + G * j, xt);
         }
     }
 #pragma unroll
@@ -126,7 +139,7 @@ k_decode_gate_up(const float *__restrict__ x, int64_t ldx, const int32_t *__rest
         return;
     }
     const int r = blockIdx.x - n_exact, slot = r / nx;
-    gate_up_rows<GT, G, UPL, PAIR, whole_gate_up(GT, G, UPL)>(x + (int64_t)(slot / n_used) * ldx, slot, r - slot * nx, idx[slot], ew, K, F,
+    gate_up_rows<GT, G, UPL, PAIR, whole_gate_up(GT, G, UPL), masks_gate_up(UPL)>(x + (int64_t)(slot / n_used) * ldx, slot, r - slot * nx, idx[slot], ew, K, F,
                                    which, h);
 }
 
@@ -384,7 +397,7 @@ k_decode_gate_up_sel(const float *__restrict__ x, int n_used, ExpertWeights ew, 
     const int e = certified ? sel_s[1 + kk]
                             : cert_select_tokens<1>(x, K, cs.w, cs.wstride, cs.ca, ra, t, emit, sel_prod)[kk];
     const uint32_t pf = certified ? prefetch_down_rows(ew, K, n_used, e_rank, lin, nwg) : 0u;
-    gate_up_rows<GT, G, UPL, true, whole_sel(GT, G, UPL), DS3_SEL_RPW>(x + (int64_t)t * K, slot, rb, e, ew, K, F, 0, h);
+    gate_up_rows<GT, G, UPL, true, whole_sel(GT, G, UPL), true, DS3_SEL_RPW>(x + (int64_t)t * K, slot, rb, e, ew, K, F, 0, h);
     asm volatile("" ::"v"(pf));                // the prefetch loads stay
 }
 
@@ -410,8 +423,8 @@ k_decode_down(const float *__restrict__ h, const int32_t *__restrict__ idx, cons
     const uint8_t *row = wd + (size_t)j * ew.down_stride;
     float acc = 0.f;
 #pragma unroll
-    for (int i = 0; i < (UPL > 0 ? UPL : 1); i++) acc += unit_dot<DT, whole_down(DT)>(row, gl + G * i, hs);
-    for (int i = (UPL > 0 ? UPL : 1); i < F / 32 / G; i++) acc += unit_dot<DT, whole_down(DT)>(row, gl + G * i, hs);
+    for (int i = 0; i < (UPL > 0 ? UPL : 1); i++) acc += unit_dot<DT, whole_down(DT, G), masks_down(G)>(row, gl + G * i, hs);
+    for (int i = (UPL > 0 ? UPL : 1); i < F / 32 / G; i++) acc += unit_dot<DT, whole_down(DT, G), masks_down(G)>(row, gl + G * i, hs);
     acc = group_sum<G>(acc);
     if (gl == 0) part[k * rows_per_wg + grp] = acc;
     __syncthreads();

@@ -684,10 +684,10 @@ def test_decode_row_dots(hip_ready, gt, dt, n_embd, n_ff):
 
 
 def decode_kernel_us(gt, dt, n_embd, n_ff, T, kernel):
-    """Best of five mean durations of one decode kernel over ten layers whose
-    expert blocks (scales and codes at random, results unread) together exceed
-    the caches."""
-    E, k, n_layers = 48, 8, 10
+    """Best of five mean durations of one decode kernel over layers whose expert
+    blocks (scales and codes at random, results unread) together exceed the
+    caches."""
+    E, k = 48, 8
     rows = ((gt, n_ff, n_embd), (gt, n_ff, n_embd), (dt, n_embd, n_ff))
     sizes = [E * r * ds3.row_bytes(t, c) for t, r, c in rows]
     noise = np.random.default_rng(1).integers(0, 256, 1 << 22, dtype=np.uint8)
@@ -698,6 +698,7 @@ def decode_kernel_us(gt, dt, n_embd, n_ff, T, kernel):
             b.write(noise[:min(noise.nbytes, n - o)], offset=o)
         return b
 
+    n_layers = max(3, (600 << 20) // sum(sizes))
     layers = [ds3.ExpertTensors(*(filled(n) for n in sizes), gt, gt, dt, n_embd, n_ff) for _ in range(n_layers)]
     router = ds3.Buffer.from_array(np.random.default_rng(2).standard_normal((E, n_embd)).astype(np.float32))
     x = ds3.Buffer.from_array(np.random.default_rng(3).standard_normal((T, n_embd)).astype(np.float32))
@@ -727,6 +728,17 @@ def test_decode_q8_rows_keep_their_loads_in_flight(hip_ready):
     b = decode_kernel_us(8, 8, 1024, 512, 2, "moe_decode_gate_up")
     print(f"  Q8_0 gate/up, T=2: 768 -> 512 {a:.1f} us, 1024 -> 512 {b:.1f} us", flush=True)
     assert a < 1.8 * b
+
+
+def test_decode_q4_long_down_rows(hip_ready):
+    """Eight tokens' Q4_K down rows, the same bytes as 512 rows of 6144 weights
+    (64 lanes per row) and as 2048 rows of 1536 (16 lanes).  The long rows take
+    about 1.1 times as long (61 against 54 us); by scale masks in place of
+    selects they took 1.7 times (92 us)."""
+    a = decode_kernel_us(12, 12, 512, 6144, 8, "moe_decode_down")
+    b = decode_kernel_us(12, 12, 2048, 1536, 8, "moe_decode_down")
+    print(f"  Q4_K down, T=8: 6144 -> 512 {a:.1f} us, 1536 -> 2048 {b:.1f} us", flush=True)
+    assert a < 1.4 * b
 
 
 def test_decode_stack_teacher_forced_config4(hip_ready):
