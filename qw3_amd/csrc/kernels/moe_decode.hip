@@ -53,8 +53,13 @@ constexpr int N_XCD_DEC = 8;   // MI355X: workgroups go round-robin to 8 XCDs
 //     Q4_K 2560 -> 1024 47 / 61)
 //   down: it wins for Q4_K up to 16 lanes (512 -> 4096, T = 4 25.0 / 22.6) and loses
 //     for Q6_K and Q8_0 (1536 -> 2048, T = 16 102 / 117 and 246 / 255)
-constexpr bool whole_gate_up(int type, int G, int UPL)
+//   one projection of mixed gate/up types: it wins for Q4_K (2048 -> 768, T = 8 25.2 /
+//     23.8; 1280 -> 1024, T = 3 16.8 / 14.3) and for Q6_K with three units up to 16
+//     lanes (1536 -> 768, T = 8 20.4 / 18.7); it loses for Q6_K else (2048 -> 768,
+//     T = 8 23.0 / 25.0) and for Q8_0 (3072 -> 1024, T = 16 144 / 162)
+constexpr bool whole_gate_up(int type, int G, int UPL, bool pair)
 {
+    if (!pair) return type == T_Q4_K || (type == T_Q6_K && UPL == 3 && G <= 16);
     return UPL == 3 && (type == T_Q4_K || (type == T_Q8_0 && G >= 16) || (type == T_Q6_K && G < 16));
 }
 constexpr bool whole_sel(int type, int G, int UPL) { return type == T_Q8_0 && UPL == 1 && G < 64; }
@@ -64,13 +69,14 @@ constexpr bool whole_down(int type, int G) { return type == T_Q4_K && G <= 16; }
 // selects (MI355X, kernel trace, us by selects / by masks):
 //   gate/up, 2-16 tokens: masks with one and three units per lane (1024 -> 3072,
 //     T = 8 71 / 68; 3072 -> 1024, T = 8 102 / 66), selects with a runtime count
-//     (2560 -> 1024, T = 4 41 / 43)
+//     (2560 -> 1024, T = 4 41 / 43); masks for one projection of mixed types (1280 ->
+//     1024, T = 4 17.0 / 14.3)
 //   down: masks up to 16 lanes per row (768 -> 2048, T = 8 30.9 / 27.9), selects
 //     above (1024 -> 3072, T = 8 61 / 66; 3072 -> 1024, T = 4 31.5 / 39.7; 6144 -> 512, T = 8
 //     61 / 92)
 // The fused selection's rows take masks throughout (768 -> 512 27.9 / 22.2, 4096 ->
 // 512 26.9 / 25.7, 1280 -> 3072 38.8 / 41.2).
-constexpr bool masks_gate_up(int UPL) { return UPL > 0; }
+constexpr bool masks_gate_up(int UPL, bool pair) { return UPL > 0 || !pair; }
 constexpr bool masks_down(int G) { return G <= 16; }
 
 // PAIR: h = swiglu(gate, up).  !PAIR: h = gate projection only, with expert
@@ -139,8 +145,8 @@ k_decode_gate_up(const float *__restrict__ x, int64_t ldx, const int32_t *__rest
         return;
     }
     const int r = blockIdx.x - n_exact, slot = r / nx;
-    gate_up_rows<GT, G, UPL, PAIR, whole_gate_up(GT, G, UPL), masks_gate_up(UPL)>(x + (int64_t)(slot / n_used) * ldx, slot, r - slot * nx, idx[slot], ew, K, F,
-                                   which, h);
+    gate_up_rows<GT, G, UPL, PAIR, whole_gate_up(GT, G, UPL, PAIR), masks_gate_up(UPL, PAIR)>(
+        x + (int64_t)(slot / n_used) * ldx, slot, r - slot * nx, idx[slot], ew, K, F, which, h);
 }
 
 // ---------------------------------------------------------------------------
