@@ -74,9 +74,10 @@ constexpr bool whole_down(int type, int G) { return type == T_Q4_K && G <= 16; }
 //   down: masks up to 16 lanes per row (768 -> 2048, T = 8 30.9 / 27.9), selects
 //     above (1024 -> 3072, T = 8 61 / 66; 3072 -> 1024, T = 4 31.5 / 39.7; 6144 -> 512, T = 8
 //     61 / 92)
-// The fused selection's rows take masks throughout (768 -> 512 27.9 / 22.2, 4096 ->
-// 512 26.9 / 25.7, 1280 -> 3072 38.8 / 41.2).
+//   gate/up with the selection: masks (768 -> 512 27.9 / 22.2, 4096 -> 512 26.9 /
+//     25.7), but selects with a runtime count at 8 lanes (1280 -> 3072 38.8 / 41.2)
 constexpr bool masks_gate_up(int UPL, bool pair) { return UPL > 0 || !pair; }
+constexpr bool masks_sel(int G, int UPL) { return UPL > 0 || G > 8; }
 constexpr bool masks_down(int G) { return G <= 16; }
 
 // PAIR: h = swiglu(gate, up).  !PAIR: h = gate projection only, with expert
@@ -403,7 +404,8 @@ k_decode_gate_up_sel(const float *__restrict__ x, int n_used, ExpertWeights ew, 
     const int e = certified ? sel_s[1 + kk]
                             : cert_select_tokens<1>(x, K, cs.w, cs.wstride, cs.ca, ra, t, emit, sel_prod)[kk];
     const uint32_t pf = certified ? prefetch_down_rows(ew, K, n_used, e_rank, lin, nwg) : 0u;
-    gate_up_rows<GT, G, UPL, true, whole_sel(GT, G, UPL), true, DS3_SEL_RPW>(x + (int64_t)t * K, slot, rb, e, ew, K, F, 0, h);
+    gate_up_rows<GT, G, UPL, true, whole_sel(GT, G, UPL), masks_sel(G, UPL), DS3_SEL_RPW>(
+        x + (int64_t)t * K, slot, rb, e, ew, K, F, 0, h);
     asm volatile("" ::"v"(pf));                // the prefetch loads stay
 }
 
