@@ -340,6 +340,17 @@ int ds3_hip_debug_grouped_lists(int32_t *meta, int32_t *counts, int32_t *offsets
  * -1 when no grouped call ran since the workspace last moved. */
 int ds3_hip_debug_grouped_descs(int32_t *desc_gu, int32_t *desc_dn);
 
+/* No ds3_metal.h counterpart (a test hook): the kernel and grid that
+ * ds3_hip_matmul_quantized_batch, or for M = 1 ds3_hip_vec_matmul_*, takes for
+ * these arguments.  plan = { kernel (0 general, 1 one-token chunked, 2 fp32
+ * MFMA, 3 fp16 MFMA), workgroups in x and y (0 for kernel 1, which sizes its
+ * grid from the device), threads per workgroup, rows of A per workgroup
+ * (kernel 2: blocks of 16; kernel 3 instead: sets of 128 rows of W) }.
+ * Launches nothing and needs no device; -1 for arguments that no product
+ * takes. */
+int ds3_hip_debug_product_plan(ds3_hip_type_t type, uint32_t M, uint32_t N, uint32_t K, uint64_t weight_row_stride,
+                               uint64_t weight_offset, int64_t *plan);
+
 /* No ds3_metal.h counterpart: the row count of A from which
  * ds3_hip_matmul_quantized_batch takes its fp16 MFMA path (see there).  0
  * restores the default (64).  Returns the previous value. */

@@ -706,6 +706,12 @@ extern "C" int ds3_hip_vec_matmul_q6k_simd(const ds3_hip_buffer_t *x, const ds3_
     return ds3_hip_vec_matmul_quantized(x, W, y, in_dim, out_dim, row_stride, T_Q6_K);
 }
 
+// matmul_quantized_batch's products with fp16 operands
+static bool dense_fp16(int type, uint32_t M, uint32_t N, uint32_t K)
+{
+    return (int64_t)M >= g.dense_mfma_min && dense_mfma_shape_ok(type, (int)N, (int)K) && M <= 65535;
+}
+
 // reference src/ds3_metal.m:2741-2828
 extern "C" int ds3_hip_matmul_quantized_batch(const ds3_hip_buffer_t *A, const ds3_hip_buffer_t *W,
                                               ds3_hip_buffer_t *C, uint32_t M, uint32_t N, uint32_t K,
@@ -736,7 +742,7 @@ extern "C" int ds3_hip_matmul_quantized_batch(const ds3_hip_buffer_t *A, const d
                 (unsigned long long)weight_row_stride);
         return -1;
     }
-    if ((int64_t)M >= g.dense_mfma_min && dense_mfma_shape_ok(type, (int)N, (int)K) && M <= 65535) {
+    if (dense_fp16(type, M, N, K)) {
         // fp16 MFMA path: A in fp16, the weights decoded to fp16, fp32 accumulate
         uint8_t *ws = ws_get((size_t)M * K * 2);
         if (!ws) return -1;
@@ -1679,6 +1685,25 @@ extern "C" int ds3_hip_debug_grouped_descs(int32_t *desc_gu, int32_t *desc_dn)
         return -1;
     if (desc_dn && n[1] > 0 && hipMemcpy(desc_dn, o.desc_dn, (size_t)n[1] * 8, hipMemcpyDeviceToHost) != hipSuccess)
         return -1;
+    return 0;
+}
+
+extern "C" int ds3_hip_debug_product_plan(ds3_hip_type_t type, uint32_t M, uint32_t N, uint32_t K,
+                                          uint64_t weight_row_stride, uint64_t weight_offset, int64_t *plan)
+{
+    if (!plan || M == 0 || N == 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || !gemv_type_ok(type, (int)K))
+        return -1;
+    if (dense_fp16(type, M, N, K)) {
+        plan[0] = 3;
+        plan[4] = dense_mfma_sets((int)M, (int)N, plan[1]);
+        plan[2] = 1;
+        plan[3] = 512;
+        return 0;
+    }
+    const GemvPlan p = gemv_plan(type, (const uint8_t *)(uintptr_t)weight_offset, weight_row_stride, (int)M, (int)N,
+                                 (int)K, nullptr);
+    const int64_t v[5] = { p.kernel, p.gx, p.gy, p.tpb, p.m_tile };
+    memcpy(plan, v, sizeof v);
     return 0;
 }
 

@@ -376,17 +376,24 @@ static hipError_t gemv_type(int G, dim3 grid, size_t lds, hipStream_t s, const f
     return hipGetLastError();
 }
 
-template <int TYPE>
-static hipError_t gemm32_type(const float *A, int64_t lda, const uint8_t *w, uint64_t stride, float *C, int64_t ldc,
-                              int M, int N, int K, hipStream_t s)
+// k_gemm32's grid: as many rows of A per workgroup as leave two workgroups
+// per CU.
+static GemvPlan gemm32_plan(int M, int N, int K)
 {
-    const int nt = (N + G32_TILE - 1) / G32_TILE, steps = K / G32_STEP;
-    const int nw = steps < G32_MAX_WAVES ? steps : G32_MAX_WAVES;
-    // as many rows of A per workgroup as leave two workgroups per CU
+    const int64_t nt = ((int64_t)N + G32_TILE - 1) / G32_TILE;
+    const int steps = K / G32_STEP;
     int mb = 4;
-    while (mb > 1 && (M <= G32_TILE * mb / 2 || (int64_t)nt * ((M + G32_TILE * mb - 1) / (G32_TILE * mb)) < 512)) mb /= 2;
-    const dim3 grid((unsigned)nt, (unsigned)((M + G32_TILE * mb - 1) / (G32_TILE * mb))), block(WAVE * nw);
-    switch (mb) {
+    while (mb > 1 && (M <= G32_TILE * mb / 2 || nt * ((M + G32_TILE * mb - 1) / (G32_TILE * mb)) < 512)) mb /= 2;
+    return { GEMV_MFMA, (unsigned)nt, (unsigned)((M + G32_TILE * mb - 1) / (G32_TILE * mb)),
+             (unsigned)(WAVE * (steps < G32_MAX_WAVES ? steps : G32_MAX_WAVES)), mb, G32_TILE };
+}
+
+template <int TYPE>
+static hipError_t gemm32_type(const GemvPlan &p, const float *A, int64_t lda, const uint8_t *w, uint64_t stride,
+                              float *C, int64_t ldc, int M, int N, int K, hipStream_t s)
+{
+    const dim3 grid(p.gx, p.gy), block(p.tpb);
+    switch (p.m_tile) {
     case 1: hipLaunchKernelGGL((k_gemm32<TYPE, 1>), grid, block, 0, s, A, lda, w, stride, C, ldc, M, N, K); break;
     case 2: hipLaunchKernelGGL((k_gemm32<TYPE, 2>), grid, block, 0, s, A, lda, w, stride, C, ldc, M, N, K); break;
     default: hipLaunchKernelGGL((k_gemm32<TYPE, 4>), grid, block, 0, s, A, lda, w, stride, C, ldc, M, N, K); break;
@@ -407,6 +414,10 @@ static hipError_t gemm32_type(const float *A, int64_t lda, const uint8_t *w, uin
 static bool gemm32_ok(int type, int M, int N, int K, const float *wnorm2)
 {
     if (wnorm2 != nullptr || K % G32_STEP != 0 || (type != T_Q4_K && type != T_Q6_K && type != T_Q8_0)) return false;
+    // a launch takes fewer than 2^32 threads in x, which 2^27 rows of W reach
+    // with 8 waves per 16 rows; k_gemv's workgroups take any number of rows
+    const GemvPlan p = gemm32_plan(M, N, K);
+    if ((uint64_t)p.gx * p.tpb >= 1ull << 32) return false;
     return M >= 2 || (N >= 2048 && K % (2 * G32_STEP) == 0);
 }
 
@@ -419,20 +430,11 @@ static int lanes_per_row(int units)
     return g;
 }
 
-hipError_t launch_gemv(int type, const float *A, int64_t lda, const uint8_t *w, uint64_t stride,
-                       float *C, int64_t ldc, int M, int N, int K, float *wnorm2, hipStream_t s)
+GemvPlan gemv_plan(int type, const uint8_t *w, uint64_t stride, int M, int N, int K, const float *wnorm2)
 {
-    if (!gemv_type_ok(type, K) || M <= 0 || N <= 0) return hipErrorInvalidValue;
-    if (gemv1_ok(type, w, stride, M, K, wnorm2)) return launch_gemv1(type, A, w, C, N, K, s);
-    if (gemm32_ok(type, M, N, K, wnorm2)) {
-        switch (type) {
-        case T_Q8_0: return gemm32_type<T_Q8_0>(A, lda, w, stride, C, ldc, M, N, K, s);
-        case T_Q4_K: return gemm32_type<T_Q4_K>(A, lda, w, stride, C, ldc, M, N, K, s);
-        default:     return gemm32_type<T_Q6_K>(A, lda, w, stride, C, ldc, M, N, K, s);
-        }
-    }
-    const int G = lanes_per_row(K / 32);
-    const int gpw = WAVE / G;
+    if (gemv1_ok(type, w, stride, M, K, wnorm2)) return { GEMV_ONE, 0, 0, G1_TPB, 1, 0 };
+    if (gemm32_ok(type, M, N, K, wnorm2)) return gemm32_plan(M, N, K);
+    const int gpw = WAVE / lanes_per_row(K / 32);
     const int rows_step = (GEMV_TPB / WAVE) * gpw;            // rows one pass of the WG covers
     int mt = GEMV_MT;
     while (mt > 1 && (size_t)mt * K * sizeof(float) > 64 * 1024) mt /= 2;
@@ -444,7 +446,24 @@ hipError_t launch_gemv(int type, const float *A, int64_t lda, const uint8_t *w, 
     int steps_per_wg = (steps_total + want_x - 1) / want_x;
     if (steps_per_wg < 1) steps_per_wg = 1;
     const int rpw = steps_per_wg * rows_step;
-    const dim3 grid((unsigned)((N + rpw - 1) / rpw), (unsigned)gy);
+    return { GEMV_GENERAL, (unsigned)((N + rpw - 1) / rpw), (unsigned)gy, GEMV_TPB, mt, rpw };
+}
+
+hipError_t launch_gemv(int type, const float *A, int64_t lda, const uint8_t *w, uint64_t stride,
+                       float *C, int64_t ldc, int M, int N, int K, float *wnorm2, hipStream_t s)
+{
+    if (!gemv_type_ok(type, K) || M <= 0 || N <= 0) return hipErrorInvalidValue;
+    const GemvPlan p = gemv_plan(type, w, stride, M, N, K, wnorm2);
+    if (p.kernel == GEMV_ONE) return launch_gemv1(type, A, w, C, N, K, s);
+    if (p.kernel == GEMV_MFMA) {
+        switch (type) {
+        case T_Q8_0: return gemm32_type<T_Q8_0>(p, A, lda, w, stride, C, ldc, M, N, K, s);
+        case T_Q4_K: return gemm32_type<T_Q4_K>(p, A, lda, w, stride, C, ldc, M, N, K, s);
+        default:     return gemm32_type<T_Q6_K>(p, A, lda, w, stride, C, ldc, M, N, K, s);
+        }
+    }
+    const int G = lanes_per_row(K / 32), mt = p.m_tile, rpw = p.rows_per_wg;
+    const dim3 grid(p.gx, p.gy);
     const size_t lds = (size_t)mt * K * sizeof(float);
     switch (type) {
     case T_F32:  return gemv_type<T_F32>(G, grid, lds, s, A, lda, w, stride, C, ldc, M, N, K, mt, rpw, wnorm2);

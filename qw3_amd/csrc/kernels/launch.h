@@ -28,6 +28,17 @@ hipError_t launch_gemv(int type, const float *A, int64_t lda, const uint8_t *w, 
                        float *C, int64_t ldc, int M, int N, int K, float *wnorm2, hipStream_t s);
 
 bool gemv_type_ok(int type, int K);
+// launch_gemv's choice for a shape that gemv_type_ok takes: the kernel
+// (k_gemv, k_gemv1, k_gemm32), its grid (not set for k_gemv1, which sizes it
+// from the device) and block, rows of A per workgroup (k_gemm32: blocks of 16)
+// and rows of W per workgroup.
+enum : int { GEMV_GENERAL = 0, GEMV_ONE = 1, GEMV_MFMA = 2 };
+struct GemvPlan {
+    int kernel;
+    unsigned gx, gy, tpb;
+    int m_tile, rows_per_wg;
+};
+GemvPlan gemv_plan(int type, const uint8_t *w, uint64_t stride, int M, int N, int K, const float *wnorm2);
 // Whether launch_gemv takes its one-token chunked path (k_gemv1) for these
 // arguments: M = 1, Q4_K / Q6_K / Q8_0, K = 2048 or 4096, dense rows, w
 // 16-byte aligned, no wnorm2.
@@ -211,6 +222,8 @@ void grouped_runs_per_tile(int n_embd, int n_ff, int S, int E, int &rpi_gu, int 
 // gate_up K loop: x16 = A [M][K] in fp16, W rows stride bytes apart.
 // Shapes: dense_mfma_shape_ok.
 bool dense_mfma_shape_ok(int type, int N, int K);
+// Sets of 128 rows of W per workgroup (1 or 2) and the grid of that choice.
+int dense_mfma_sets(int M, int N, int64_t &grid);
 hipError_t launch_dense_mfma(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int type, int M, int N,
                              float *c, hipStream_t s);
 

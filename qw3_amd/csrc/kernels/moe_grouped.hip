@@ -966,9 +966,7 @@ hipError_t launch_grouped_gate_up(const _Float16 *x16, int K, const ExpertWeight
     }
 }
 
-template <int TV>
-static hipError_t dense_t(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int M, int N, float *c,
-                          hipStream_t s)
+int dense_mfma_sets(int M, int N, int64_t &grid)
 {
     const int64_t m_tiles = (M + GG_TILE_M - 1) / GG_TILE_M, t2 = m_tiles * (N / (2 * GG_TILE_N));
     const int64_t n_cu = device_cu_count();
@@ -981,14 +979,24 @@ static hipError_t dense_t(const _Float16 *x16, int K, const uint8_t *w, uint64_t
     // 41.9; 600 x 2048 -> 8192 (2 / 3) 52.2 / 48.6 | 75.0 / 61.4 | 76.3 / 60.7;
     // 1024 x 2048 -> 8192 (2 / 4) 58.3 / 68.0 | 79.8 / 84.5 | 81.6 / 84.3.
     const bool one = 2 * ((2 * t2 + n_cu - 1) / n_cu) <= 3 * ((t2 + n_cu - 1) / n_cu);
-    const int64_t grid = ((one ? 2 * t2 : t2) + N_XCD - 1) / N_XCD * N_XCD;
+    grid = ((one ? 2 * t2 : t2) + N_XCD - 1) / N_XCD * N_XCD;
+    return one ? 1 : 2;
+}
+
+template <int TV>
+static hipError_t dense_t(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int M, int N, float *c,
+                          hipStream_t s)
+{
+    int64_t grid;
+    const bool one = dense_mfma_sets(M, N, grid) == 1;
+    const int m_tiles = (M + GG_TILE_M - 1) / GG_TILE_M;
     if (grid > INT32_MAX / 2) return hipErrorInvalidValue;
     if (one)
         hipLaunchKernelGGL((k_dense<TV, 1>), dim3((unsigned)grid), dim3(64 * GG_WV), 0, s, x16, K, w, stride, M, N,
-                           (int)m_tiles, c);
+                           m_tiles, c);
     else
         hipLaunchKernelGGL((k_dense<TV, 2>), dim3((unsigned)grid), dim3(64 * GG_WV), 0, s, x16, K, w, stride, M, N,
-                           (int)m_tiles, c);
+                           m_tiles, c);
     return hipGetLastError();
 }
 

@@ -90,3 +90,25 @@ def test_capture_refusals(capfd):
                  "router_stats", "timer_start", "graph_launch"):
         assert f"{what}" in err and "not allowed during graph capture" in err, what
     assert err.count("not allowed during graph capture") >= 8
+
+
+def product_plan(t, M, N, K, pad=0, offset=0):
+    """(kernel, grid x, grid y, threads, tile) that a dense product takes."""
+    lib = _native._bind(C.CDLL(str(_native.LIB_DIR / "libds3_hip.so")), _native.SIGNATURES)
+    plan = (C.c_int64 * 5)()
+    per, nbytes = {12: (256, 144), 14: (256, 210), 8: (32, 34)}[t]
+    assert lib.ds3_hip_debug_product_plan(t, M, N, K, K // per * nbytes + pad, offset, plan) == 0, (t, M, N, K)
+    return tuple(plan)
+
+
+def test_product_grids_fit_a_launch():
+    """A launch takes fewer than 2^32 threads in x and 2^16 workgroups in y: every
+    product whose operands 288 GB can hold has a kernel whose grid fits."""
+    for t in (12, 14, 8):
+        for K in (256, 512, 1024, 2048, 4096):
+            for N in (1, 2048, (1 << 27) - 16, 1 << 27, (1 << 27) + 1, 1 << 28, 1 << 29, 1 << 30):
+                for M in (1, 2, 40, 1000):
+                    if N * K // 256 * {12: 144, 14: 210, 8: 272}[t] + 4 * M * N > 288e9:
+                        continue
+                    kernel, gx, gy, threads, tile = product_plan(t, M, N, K, pad=8)
+                    assert gx * threads < 1 << 32 and gy < 1 << 16, (t, M, N, K, kernel, gx, gy, threads)
