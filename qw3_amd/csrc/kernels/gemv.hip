@@ -401,16 +401,26 @@ static hipError_t gemm32_type(const GemvPlan &p, const float *A, int64_t lda, co
     return hipGetLastError();
 }
 
-// k_gemm32's shapes: quantised rows of whole 256-wide steps.  From two rows of
-// A it always wins (MI355X, k_gemv against k_gemm32, Q4_K / Q6_K / Q8_0: 2 x
-// 2048 -> 768 10.2 / 8.6 / 13.6 against 7.0 / 7.6 / 6.6 us; 63 x 512 -> 300
-// 13.5 / 11.2 / 20.5 against 6.5 / 6.5 / 5.5 us).  One row fills 1/16 of the
-// tile but still decodes faster with every lane group on its own unit: 1024 ->
-// 20,000 26.3 / 18.1 / 44.2 against 11.0 / 12.9 / 10.5 us, 512 -> 131,072 47.5
-// / 39.0 / 77.8 against 29.4 / 35.3 / 30.3, 1024 -> 4096 8.0 / 6.4 / 11.5
-// against 6.5 / 6.4 / 6.4.  One row stays on k_gemv below 2048 rows of W (1024
-// -> 700 5.9 / 5.6 against 6.4 / 6.5 us in Q4_K / Q6_K) and at an odd number
-// of steps (768 -> 32,000 11.2 / 11.1 against 13.8 / 16.2 us).
+// k_gemm32's shapes: quantised rows of whole 256-wide steps, wherever it beats
+// k_gemv.  Measured on MI355X, us per call back to back, k_gemv / k_gemm32:
+//   3 rows of A and more: it wins (3 x 256 -> 64 4.7 / 4.2 in Q4_K, 27 x 2048 ->
+//     768 73 / 7.6; the worst is Q6_K 3 x 1280 -> 16,384, 1.08 times)
+//   2 rows: it wins (2 x 2048 -> 768 10.2 / 7.0, 8.6 / 7.6, 13.6 / 6.6 in Q4_K, Q6_K,
+//     Q8_0) but for K = 256 in Q4_K and Q6_K, where a workgroup is one wave (-> 768
+//     4.1 / 4.5; -> 12,288 in Q4_K 0.84 times, -> 24,000 in Q6_K 0.89), and Q6_K at
+//     K = 1280, whose five waves share four SIMDs (-> 32,000 26.3 / 28.6)
+//   one row fills 1/16 of a tile, but every lane group decodes its own unit.
+//     Below 2048 rows of W (1024 -> 700 5.9 / 6.4) and at an odd number of steps
+//     (768 -> 32,000 11.2 / 13.8) k_gemv wins.
+//     Q8_0: it wins (512 -> 4096 4.9 / 4.3, 1024 -> 20,000 44 / 10.0)
+//     Q4_K: it wins (1024 -> 20,000 26 / 9.8, 1536 -> 4096 7.6 / 5.3), at K = 512
+//       from 12,288 rows (0.69 times; -> 8192 5.3 / 5.4)
+//     Q6_K: its decode costs more.  It wins where K / 32 units are whole turns of
+//       32 lanes and more than half the CUs get a tile (1024 -> 4096 5.9 / 5.0; ->
+//       2048 4.7 / 5.0), else up to one tile a CU (1536 -> 4096 7.0 / 6.2; -> 8192
+//       8.0 / 9.8, -> 100,000 76 / 92; past one tile a CU the two cross several
+//       times, with 2560 -> 20,000 32 / 28 the other way), at K = 512 from 12,288
+//       rows (-> 32,000 0.97 times; -> 8192 4.8 / 6.0)
 static bool gemm32_ok(int type, int M, int N, int K, const float *wnorm2)
 {
     if (wnorm2 != nullptr || K % G32_STEP != 0 || (type != T_Q4_K && type != T_Q6_K && type != T_Q8_0)) return false;
@@ -418,7 +428,17 @@ static bool gemm32_ok(int type, int M, int N, int K, const float *wnorm2)
     // with 8 waves per 16 rows; k_gemv's workgroups take any number of rows
     const GemvPlan p = gemm32_plan(M, N, K);
     if ((uint64_t)p.gx * p.tpb >= 1ull << 32) return false;
-    return M >= 2 || (N >= 2048 && K % (2 * G32_STEP) == 0);
+    if (M >= 3) return true;
+    if (M == 2) {
+        if (type == T_Q8_0) return true;
+        if (K == G32_STEP) return N >= (type == T_Q4_K ? 12288 : 24000);
+        return type != T_Q6_K || K != 5 * G32_STEP || N <= 12288;
+    }
+    if (N < 2048 || K % (2 * G32_STEP) != 0) return false;
+    if (type == T_Q8_0) return true;
+    if (K == 2 * G32_STEP) return N >= 12288;
+    if (type == T_Q4_K) return true;
+    return K % 1024 == 0 ? N > 2048 : N <= 4096;
 }
 
 // Lanes per row: the largest power of two dividing the unit count (no idle

@@ -112,3 +112,25 @@ def test_product_grids_fit_a_launch():
                         continue
                     kernel, gx, gy, threads, tile = product_plan(t, M, N, K, pad=8)
                     assert gx * threads < 1 << 32 and gy < 1 << 16, (t, M, N, K, kernel, gx, gy, threads)
+
+
+def test_product_kernel_choice():
+    """The fp32 product kernel at sizes on both sides of each line of the
+    dispatch: where the matrix-core kernel (2) measured slower than the general
+    one (0), the call keeps the general one."""
+    q4, q6, q8 = 12, 14, 8
+    want = {
+        (q6, 1, 8192, 512): 0, (q6, 1, 12288, 512): 2, (q4, 1, 8192, 512): 0, (q4, 1, 12288, 512): 2,
+        (q8, 1, 2048, 512): 2, (q8, 1, 2047, 512): 0, (q4, 1, 2048, 1024): 2, (q6, 1, 2048, 1024): 0,
+        (q6, 1, 2560, 1024): 2, (q6, 1, 4096, 1536): 2, (q6, 1, 8192, 1536): 0, (q6, 1, 100000, 1536): 0,
+        (q4, 1, 100000, 1536): 2, (q6, 1, 2048, 8192): 0, (q6, 1, 4096, 8192): 2, (q8, 1, 32000, 768): 0,
+        (q4, 2, 768, 256): 0, (q4, 2, 12288, 256): 2, (q6, 2, 12288, 256): 0, (q6, 2, 24000, 256): 2,
+        (q8, 2, 64, 256): 2, (q6, 2, 32000, 1280): 0, (q6, 2, 8192, 1280): 2, (q4, 2, 32000, 1280): 2,
+        (q6, 2, 2048, 768): 2, (q4, 3, 64, 256): 2, (q6, 3, 32000, 1280): 2, (q8, 8, 300, 288): 0,
+        (q4, 63, 768, 2048): 2, (q4, 64, 768, 2048): 3, (q4, 64, 768, 768): 2, (q6, 64, 700, 2048): 2,
+    }
+    got = {k: product_plan(*k, pad=2)[0] for k in want}
+    assert got == want
+    # dense rows of 2048 and 4096 from a 16-byte boundary run on the one-token kernel
+    assert [product_plan(q6, 1, 2048, 2048)[0], product_plan(q6, 1, 2048, 2048, offset=8)[0],
+            product_plan(q4, 1, 17, 4096)[0], product_plan(q4, 1, 17, 4096, pad=16)[0]] == [1, 0, 1, 0]
