@@ -9,6 +9,8 @@ Bars:
   - the fp16-MFMA path of matmul_quantized_batch: the north-star bar on
     outputs, relative L2 <= 1e-3, and max-abs <= 2e-3 on outputs scaled to
     unit RMS."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -32,6 +34,14 @@ def normal_matrix(t, seed, rows, cols):
 
 def kernels_run():
     return set(ds3.kernel_stats())
+
+
+def product_plan(t, M, N, K, stride, offset=0):
+    """(kernel, workgroups x and y, threads, tile) that a product takes: kernel 0
+    general, 1 one-token chunked, 2 fp32 and 3 fp16 matrix cores."""
+    plan = (C.c_int64 * 5)()
+    assert hip().ds3_hip_debug_product_plan(t, M, N, K, stride, offset, plan) == 0
+    return tuple(plan)
 
 
 @pytest.mark.parametrize("t,M,N,K", [(12, 64, 512, 2048), (12, 512, 4096, 2048), (14, 100, 2048, 4096),
@@ -66,28 +76,37 @@ def test_matmul_quantized_batch_mfma(hip_ready, t, M, N, K):
 
 
 @pytest.mark.parametrize("t", [12, 14, 8])
-@pytest.mark.parametrize("M,N,K,off", [(65, 256, 512, 0), (16, 1024, 1024, 6), (709, 3328, 512, 0), (709, 3328, 512, 2),
-                                       (64, 66048, 512, 0)])
-def test_matmul_quantized_batch_mfma_tiles(hip_ready, t, M, N, K, off):
-    """Both tile widths of the matrix-core product (128 columns while the wide
-    tiles leave the last round of CUs short, 256 for 709 x 3328), one row in the
-    last token tile, a grid rounded up to the XCDs, rows off 16 bytes, and more
-    than 65,536 columns; the bars of test_matmul_quantized_batch_mfma."""
+@pytest.mark.parametrize("M,N,K,off,pad,sets", [
+    (65, 256, 512, 0, 0, 1), (16, 1024, 1024, 6, 0, 1), (88, 256, 512, 0, 16, 1), (104, 512, 1024, 0, 6, 1),
+    (709, 3328, 512, 0, 0, 2), (709, 3328, 512, 2, 0, 2), (728, 3328, 512, 0, 0, 2), (728, 3328, 512, 2, 2, 2),
+    (744, 3328, 512, 0, 32, 2), (744, 3328, 512, 2, 0, 2), (64, 66048, 512, 0, 0, 1)])
+def test_matmul_quantized_batch_mfma_tiles(hip_ready, t, M, N, K, off, pad, sets):
+    """Both tile widths of the matrix-core product (`sets` of 128 columns: one
+    while wide tiles leave the last round of CUs short, two for 709 x 3328),
+    last token tiles of one to four 16-row blocks (704 + 5, 24 and 40 rows at
+    two sets, 64 + 1, 24 and 40 at one), a grid rounded up to the XCDs, rows off
+    16 bytes and rows padded past their bytes, and more than 65,536 columns:
+    relative L2 as in test_matmul_quantized_batch_mfma, the largest error
+    within 6 sigma of the operands' rounding."""
     A = np.random.default_rng(M + N + t).standard_normal((M, K)).astype(np.float32)
+    rb = ds3.row_bytes(t, K)
     raw = normal_matrix(t, 7, N, K)
-    want = A @ O.dequantize(t, raw, N * K).reshape(N, K).T
-    wb = ds3.Buffer.alloc(raw.nbytes + off)
-    wb.write(raw, offset=off)
+    want = A.astype(np.float64) @ O.dequantize(t, raw, N * K).reshape(N, K).astype(np.float64).T
+    rows = np.full((N, rb + pad), 255, np.uint8)              # a padding byte read as a weight would show
+    rows[:, :rb] = raw.reshape(N, rb)
+    wb = ds3.Buffer.alloc(rows.nbytes + off)
+    wb.write(rows, offset=off)
     cb = ds3.Buffer.alloc(M * N * 4)
-    print(f"  dense tiles {ds3.TYPE_NAMES[t]} M={M} N={N} K={K} offset {off}", flush=True)
+    print(f"  dense tiles {ds3.TYPE_NAMES[t]} M={M} N={N} K={K} offset {off} pad {pad}", flush=True)
     prev = hip().ds3_hip_set_dense_mfma_min_rows(16)
     try:
-        assert hip().ds3_hip_matmul_quantized_batch(ds3.Buffer.from_array(A), wb, cb, M, N, K, ds3.row_bytes(t, K),
-                                                    off, t) == 0
+        plan = product_plan(t, M, N, K, rb + pad, off)
+        assert hip().ds3_hip_matmul_quantized_batch(ds3.Buffer.from_array(A), wb, cb, M, N, K, rb + pad, off, t) == 0
     finally:
         hip().ds3_hip_set_dense_mfma_min_rows(prev)
+    assert plan[0] == 3 and plan[4] == sets
     got = cb.read(np.float32, (M, N))
-    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    rms = float(np.sqrt(np.mean(want ** 2)))
     assert O.rel_l2(got, want) <= MFMA_REL_L2
     # rounding of A and W to fp16: at most 4e-4 rms relative to the unit-rms output
     # (2^-11 / sqrt(3) each, times sqrt 2); 4.3 million outputs of one case
@@ -239,29 +258,43 @@ def test_vec_matmul_q4k_half(hip_ready):
 
 
 @pytest.mark.parametrize("t", [12, 14, 8])
-@pytest.mark.parametrize("M,N,K,shift", [(2, 1, 256, 0), (15, 17, 512, 0), (16, 768, 2048, 2), (17, 300, 768, 4),
-                                         (33, 49, 2304, 0), (63, 4112, 1024, 1), (200, 100, 4096, 0), (1, 2049, 512, 2)])
-def test_matmul_quantized_batch_few_rows(hip_ready, t, M, N, K, shift):
-    """Products below the MFMA row count (or of shapes that path does not
-    take) run in fp32 on the matrix cores: partial tiles of rows and columns, 1 to 16 K steps over up to 8 waves, A on a 4-byte boundary,
-    and weights `shift` bytes past a dword.  Each result is a chain of 32
-    products and a tree of at most 12 sums over the exact decoded weights, so
-    it lies within (32 + 12) * 2^-23 of the sum of absolute products (twice
-    the rounding unit, as the matrix core's own rounding is not specified)."""
+@pytest.mark.parametrize("M,N,K,shift,pad,blocks", [
+    (2, 1, 256, 0, 0, 0), (3, 1, 256, 0, 0, 1), (15, 17, 512, 0, 0, 1), (16, 768, 2048, 2, 0, 1), (17, 300, 768, 4, 0, 1),
+    (33, 49, 2304, 0, 0, 1), (63, 4112, 1024, 1, 0, 2), (32, 8192, 512, 0, 6, 2), (200, 100, 4096, 0, 0, 1),
+    (33, 8200, 512, 0, 0, 4), (63, 8200, 256, 3, 2, 4), (100, 4100, 768, 0, 16, 4), (1, 2049, 512, 2, 0, 0),
+    (1, 2577, 1024, 2, 0, 1)])
+def test_matmul_quantized_batch_few_rows(hip_ready, t, M, N, K, shift, pad, blocks):
+    """Products below the fp16 row count (or of shapes that path does not
+    take) run in fp32 on the matrix cores, `blocks` of 16 rows of A per
+    workgroup (0: the general kernel, which serves the smallest one- and
+    two-row products in Q4_K and Q6_K): partial tiles of rows and columns, a
+    last workgroup of 36 rows, 1 to 16 K steps over up to 8 waves, A on a 4-byte
+    boundary, weights `shift` bytes past a dword and rows padded past their
+    bytes.  Each result is a chain of 32 products and a tree of at most 12 sums
+    over the exact decoded weights, so it lies within (32 + 12) * 2^-23 of the
+    sum of absolute products (twice the rounding unit, as the matrix core's
+    own rounding is not specified)."""
     rng = np.random.default_rng(M * 7 + N + K + t)
     A = rng.standard_normal((M, K)).astype(np.float32)
+    rb = ds3.row_bytes(t, K)
     raw = normal_matrix(t, 21, N, K)
     Wf = O.dequantize(t, raw, N * K).reshape(N, K).astype(np.float64)
     want = A.astype(np.float64) @ Wf.T
     bound = 44 * 2.0 ** -23 * (np.abs(A).astype(np.float64) @ np.abs(Wf).T)
-    wb = ds3.Buffer.alloc(raw.nbytes + 16)
-    wb.write(raw, offset=shift)
+    rows = np.full((N, rb + pad), 255, np.uint8)              # a padding byte read as a weight would show
+    rows[:, :rb] = raw.reshape(N, rb)
+    wb = ds3.Buffer.alloc(rows.nbytes + 16)
+    wb.write(rows, offset=shift)
     ab = ds3.Buffer.alloc(M * K * 4 + 4)
     ab.write(A, offset=4)
     cb = ds3.Buffer.alloc(M * N * 4)
-    print(f"  few rows {ds3.TYPE_NAMES[t]} M={M} N={N} K={K} shift={shift}", flush=True)
-    assert hip().ds3_hip_matmul_quantized_batch(ab.view(4, M * K * 4), wb, cb, M, N, K, ds3.row_bytes(t, K), shift,
-                                                t) == 0
+    print(f"  few rows {ds3.TYPE_NAMES[t]} M={M} N={N} K={K} shift={shift} pad={pad}", flush=True)
+    plan = product_plan(t, M, N, K, rb + pad, shift)
+    if blocks:
+        assert plan[0] == 2 and plan[4] == blocks
+    else:
+        assert plan[0] == (2 if t == 8 else 0)
+    assert hip().ds3_hip_matmul_quantized_batch(ab.view(4, M * K * 4), wb, cb, M, N, K, rb + pad, shift, t) == 0
     err = np.abs(cb.read(np.float32, (M, N)).astype(np.float64) - want)
     print(f"    worst error / bound {float((err / bound).max()):.3f}", flush=True)
     assert (err <= bound).all()
