@@ -345,7 +345,8 @@ int ds3_hip_debug_grouped_descs(int32_t *desc_gu, int32_t *desc_dn);
  * these arguments.  plan = { kernel (0 general, 1 one-token chunked, 2 fp32
  * MFMA, 3 fp16 MFMA), workgroups in x and y (0 for kernel 1, which sizes its
  * grid from the device), threads per workgroup, rows of A per workgroup
- * (kernel 2: blocks of 16; kernel 3 instead: sets of 128 rows of W) }.
+ * (kernel 2: blocks of 16; kernel 3 instead: sets of 128 rows of W), for
+ * kernel 3 whether consecutive workgroups share rows of A and not of W }.
  * Launches nothing and needs no device; -1 for arguments that no product
  * takes. */
 int ds3_hip_debug_product_plan(ds3_hip_type_t type, uint32_t M, uint32_t N, uint32_t K, uint64_t weight_row_stride,

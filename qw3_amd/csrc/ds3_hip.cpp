@@ -1698,11 +1698,12 @@ extern "C" int ds3_hip_debug_product_plan(ds3_hip_type_t type, uint32_t M, uint3
         plan[4] = dense_mfma_sets((int)M, (int)N, plan[1]);
         plan[2] = 1;
         plan[3] = 512;
+        plan[5] = dense_mfma_a_first((int)M, (int)N, (int)K, weight_row_stride) ? 1 : 0;
         return 0;
     }
     const GemvPlan p = gemv_plan(type, (const uint8_t *)(uintptr_t)weight_offset, weight_row_stride, (int)M, (int)N,
                                  (int)K, nullptr);
-    const int64_t v[5] = { p.kernel, p.gx, p.gy, p.tpb, p.m_tile };
+    const int64_t v[6] = { p.kernel, p.gx, p.gy, p.tpb, p.m_tile, 0 };
     memcpy(plan, v, sizeof v);
     return 0;
 }

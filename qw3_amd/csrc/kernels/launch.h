@@ -224,6 +224,8 @@ void grouped_runs_per_tile(int n_embd, int n_ff, int S, int E, int &rpi_gu, int 
 bool dense_mfma_shape_ok(int type, int N, int K);
 // Sets of 128 rows of W per workgroup (1 or 2) and the grid of that choice.
 int dense_mfma_sets(int M, int N, int64_t &grid);
+// Whether consecutive tiles share rows of A and not rows of W.
+bool dense_mfma_a_first(int M, int N, int K, uint64_t stride);
 hipError_t launch_dense_mfma(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int type, int M, int N,
                              float *c, hipStream_t s);
 

@@ -840,20 +840,22 @@ k_grouped_down(const _Float16 *__restrict__ h16, int F, ExpertWeights ew, int N,
 
 // Dense C[M][N] = A[M][K] W[N][K]^T: a workgroup takes 64 rows of A and NB
 // sets of 128 rows of W (sets N / NB apart) on gate_up's K loop; its tile comes
-// from the block index, so no list launch precedes it.  Tiles of one W set are
-// consecutive on one XCD, so its weights come through one L2.  Bound by the
-// weight decode, repeated for every 64 rows of A: 512 x 2048 -> 4096 in Q4_K
-// 31.3 -> 21.8 us with the conversion of A (393 TFLOP/s; before, 256-row tiles
-// from a one-workgroup list kernel left half the CUs idle).
+// from the block index, so no list launch precedes it.  `inner` consecutive
+// tiles, on one XCD, share their W sets or, with a_first, their rows of A
+// (dense_mfma_a_first).  Bound by the weight decode, repeated for every 64 rows
+// of A: 512 x 2048 -> 4096 in Q4_K 31.3 -> 21.8 us with the conversion of A
+// (393 TFLOP/s; before, 256-row tiles from a one-workgroup list kernel left
+// half the CUs idle).
 template <int TYPE, int NB>
 __global__ void __launch_bounds__(64 * GG_WV)
 k_dense(const _Float16 *__restrict__ x16, int K, const uint8_t *__restrict__ w, uint64_t stride, int M, int N,
-        int m_tiles, float *__restrict__ c)
+        int inner, int a_first, int tiles, float *__restrict__ c)
 {
     __shared__ __attribute__((aligned(16))) uint8_t smem[2 * GG_CHUNK];
-    const int idx = gg_list_index(0), nt = idx / m_tiles;
-    if (nt >= N / (NB * GG_TILE_N)) return;              // uniform: the grid is rounded up to the XCDs
-    const int row0 = (idx - nt * m_tiles) * GG_TILE_M, mrows = min(GG_TILE_M, M - row0);
+    const int idx = gg_list_index(0);
+    if (idx >= tiles) return;                            // uniform: the grid is rounded up to the XCDs
+    const int out = idx / inner, in = idx - out * inner, nt = a_first ? in : out, mt = a_first ? out : in;
+    const int row0 = mt * GG_TILE_M, mrows = min(GG_TILE_M, M - row0);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t a_lds = (uint32_t)(uintptr_t)(DS3_LDS void *)smem;
     uint32_t lofs[8];
@@ -983,20 +985,26 @@ int dense_mfma_sets(int M, int N, int64_t &grid)
     return one ? 1 : 2;
 }
 
+// Whether consecutive tiles share rows of A and not rows of W.  An XCD streams
+// all of the operand whose tiles vary fastest and its own eighth of the other,
+// so the larger one varies slowest.  MI355X, us per call with W / A shared:
+// 4096 x 512 -> 4096 in Q4_K 53.9 / 41.2, 2048 x 2048 -> 4096 62.5 / 55.9, 4096 x
+// 512 -> 1024 19.3 / 15.5; 512 x 512 -> 16,384 22.8 / 27.0, 1000 x 512 -> 8192 in
+// Q8_0 28.4 / 31.6.
+bool dense_mfma_a_first(int M, int N, int K, uint64_t stride) { return (uint64_t)M * K * 2 > (uint64_t)N * stride; }
+
 template <int TV>
 static hipError_t dense_t(const _Float16 *x16, int K, const uint8_t *w, uint64_t stride, int M, int N, float *c,
                           hipStream_t s)
 {
     int64_t grid;
-    const bool one = dense_mfma_sets(M, N, grid) == 1;
-    const int m_tiles = (M + GG_TILE_M - 1) / GG_TILE_M;
+    const int sets = dense_mfma_sets(M, N, grid);
     if (grid > INT32_MAX / 2) return hipErrorInvalidValue;
-    if (one)
-        hipLaunchKernelGGL((k_dense<TV, 1>), dim3((unsigned)grid), dim3(64 * GG_WV), 0, s, x16, K, w, stride, M, N,
-                           m_tiles, c);
-    else
-        hipLaunchKernelGGL((k_dense<TV, 2>), dim3((unsigned)grid), dim3(64 * GG_WV), 0, s, x16, K, w, stride, M, N,
-                           m_tiles, c);
+    const int m_tiles = (M + GG_TILE_M - 1) / GG_TILE_M, n_tiles = N / (sets * GG_TILE_N);
+    const bool a_first = dense_mfma_a_first(M, N, K, stride);
+    const auto kernel = sets == 1 ? k_dense<TV, 1> : k_dense<TV, 2>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * GG_WV), 0, s, x16, K, w, stride, M, N,
+                       a_first ? n_tiles : m_tiles, a_first ? 1 : 0, m_tiles * n_tiles, c);
     return hipGetLastError();
 }
 

@@ -93,9 +93,9 @@ def test_capture_refusals(capfd):
 
 
 def product_plan(t, M, N, K, pad=0, offset=0):
-    """(kernel, grid x, grid y, threads, tile) that a dense product takes."""
+    """(kernel, grid x, grid y, threads, tile, order) that a dense product takes."""
     lib = _native._bind(C.CDLL(str(_native.LIB_DIR / "libds3_hip.so")), _native.SIGNATURES)
-    plan = (C.c_int64 * 5)()
+    plan = (C.c_int64 * 6)()
     per, nbytes = {12: (256, 144), 14: (256, 210), 8: (32, 34)}[t]
     assert lib.ds3_hip_debug_product_plan(t, M, N, K, K // per * nbytes + pad, offset, plan) == 0, (t, M, N, K)
     return tuple(plan)
@@ -110,7 +110,7 @@ def test_product_grids_fit_a_launch():
                 for M in (1, 2, 40, 1000):
                     if N * K // 256 * {12: 144, 14: 210, 8: 272}[t] + 4 * M * N > 288e9:
                         continue
-                    kernel, gx, gy, threads, tile = product_plan(t, M, N, K, pad=8)
+                    kernel, gx, gy, threads, _, _ = product_plan(t, M, N, K, pad=8)
                     assert gx * threads < 1 << 32 and gy < 1 << 16, (t, M, N, K, kernel, gx, gy, threads)
 
 
@@ -134,3 +134,8 @@ def test_product_kernel_choice():
     # dense rows of 2048 and 4096 from a 16-byte boundary run on the one-token kernel
     assert [product_plan(q6, 1, 2048, 2048)[0], product_plan(q6, 1, 2048, 2048, offset=8)[0],
             product_plan(q4, 1, 17, 4096)[0], product_plan(q4, 1, 17, 4096, pad=16)[0]] == [1, 0, 1, 0]
+    # the fp16 product's tile order: the larger operand's tiles vary slowest (A 2 bytes a
+    # weight, W 0.5625 in Q4_K and 1.0625 in Q8_0)
+    assert [product_plan(t, M, N, 512)[5] for t, M, N in ((q4, 4096, 4096), (q4, 4096, 5120), (q4, 512, 16384),
+                                                         (q8, 1000, 8192), (q8, 3000, 4096), (q4, 512, 4096))] == \
+        [1, 1, 0, 0, 1, 0]

@@ -37,9 +37,9 @@ def kernels_run():
 
 
 def product_plan(t, M, N, K, stride, offset=0):
-    """(kernel, workgroups x and y, threads, tile) that a product takes: kernel 0
-    general, 1 one-token chunked, 2 fp32 and 3 fp16 matrix cores."""
-    plan = (C.c_int64 * 5)()
+    """(kernel, workgroups x and y, threads, tile, order) that a product takes:
+    kernel 0 general, 1 one-token chunked, 2 fp32 and 3 fp16 matrix cores."""
+    plan = (C.c_int64 * 6)()
     assert hip().ds3_hip_debug_product_plan(t, M, N, K, stride, offset, plan) == 0
     return tuple(plan)
 
@@ -77,6 +77,7 @@ def test_matmul_quantized_batch_mfma(hip_ready, t, M, N, K):
 
 @pytest.mark.parametrize("t", [12, 14, 8])
 @pytest.mark.parametrize("M,N,K,off,pad,sets", [
+    (333, 256, 512, 2, 0, 1), (1993, 1280, 512, 0, 16, 2), (1993, 1280, 512, 2, 0, 2),       # A the larger operand
     (65, 256, 512, 0, 0, 1), (16, 1024, 1024, 6, 0, 1), (88, 256, 512, 0, 16, 1), (104, 512, 1024, 0, 6, 1),
     (709, 3328, 512, 0, 0, 2), (709, 3328, 512, 2, 0, 2), (728, 3328, 512, 0, 0, 2), (728, 3328, 512, 2, 2, 2),
     (744, 3328, 512, 0, 32, 2), (744, 3328, 512, 2, 0, 2), (64, 66048, 512, 0, 0, 1)])
@@ -84,8 +85,8 @@ def test_matmul_quantized_batch_mfma_tiles(hip_ready, t, M, N, K, off, pad, sets
     """Both tile widths of the matrix-core product (`sets` of 128 columns: one
     while wide tiles leave the last round of CUs short, two for 709 x 3328),
     last token tiles of one to four 16-row blocks (704 + 5, 24 and 40 rows at
-    two sets, 64 + 1, 24 and 40 at one), a grid rounded up to the XCDs, rows off
-    16 bytes and rows padded past their bytes, and more than 65,536 columns:
+    two sets, 64 + 1, 24 and 40 at one), both orders of the tiles, a grid rounded
+    up to the XCDs, rows off 16 bytes and rows padded past their bytes, and more than 65,536 columns:
     relative L2 as in test_matmul_quantized_batch_mfma, the largest error
     within 6 sigma of the operands' rounding."""
     A = np.random.default_rng(M + N + t).standard_normal((M, K)).astype(np.float32)
@@ -105,6 +106,8 @@ def test_matmul_quantized_batch_mfma_tiles(hip_ready, t, M, N, K, off, pad, sets
     finally:
         hip().ds3_hip_set_dense_mfma_min_rows(prev)
     assert plan[0] == 3 and plan[4] == sets
+    if M in (333, 1993, 709):
+        assert plan[5] == (M != 709)
     got = cb.read(np.float32, (M, N))
     rms = float(np.sqrt(np.mean(want ** 2)))
     assert O.rel_l2(got, want) <= MFMA_REL_L2
