@@ -35,8 +35,14 @@ bool gemv_type_ok(int type, int K);
 #ifndef DS3_G1_ROWS
 #define DS3_G1_ROWS 4               // rows per chunk at K = 2048 (half at 4096, at least 4)
 #endif
+// Persistent workgroups per CU.  6, but 3 for Q8_0 rows of 2048: of 6 five fit at
+// once (87 VGPRs), and the sixth's share of the chunks runs after them alone;
+// with 3 they all run, with as many bytes in flight as the memory needs.  MI355X, us
+// per call with 3 / 5 / 6 on weights that come from memory: Q8_0 2048 -> 151,936
+// 59.3 / 62.4 / 66.3, -> 20,000 12.2 / 13.8 / 15.6; 4096 -> 300,000 229 / 227 / 229;
+// Q4_K 2048 -> 151,936 48.4 / 45.3 / 44.8; Q6_K 55.9 / 57.6 / 55.3.
 #ifndef DS3_G1_WPC
-#define DS3_G1_WPC 6                // persistent workgroups per CU
+#define DS3_G1_WPC 6
 #endif
 #ifndef DS3_G1_SETS
 #define DS3_G1_SETS 2               // register sets of chunks in flight per workgroup
@@ -119,7 +125,8 @@ static hipError_t gemv1_t(const float *x, const uint8_t *w, float *y, int N, hip
             n_cu = 256;
     }
     const int nch = (N + G1<TYPE, UPL>::R - 1) / G1<TYPE, UPL>::R;
-    const int grid = nch < DS3_G1_WPC * n_cu ? nch : DS3_G1_WPC * n_cu;
+    constexpr int wpc = TYPE == T_Q8_0 && UPL == 1 ? 3 : DS3_G1_WPC;
+    const int grid = nch < wpc * n_cu ? nch : wpc * n_cu;
     hipLaunchKernelGGL((k_gemv1<TYPE, UPL>), dim3((unsigned)grid), dim3(G1_TPB), 0, s, x, w, y, N, nch);
     return hipGetLastError();
 }
