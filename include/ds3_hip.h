@@ -100,11 +100,14 @@ int ds3_hip_vec_matmul_q4k_half(const ds3_hip_buffer_t *x, const ds3_hip_buffer_
 
 /* reference src/ds3_metal.h:154-161: C[M][N] = A[M][K] . W[N][K]^T, fp32,
  * W at byte weight_offset inside the buffer.  Below the dense-MFMA row
- * count (ds3_hip_set_dense_mfma_min_rows, default 64) every product is an
- * fp32 FMA on the exactly decoded weights, as the reference's kernel
- * computes.  From that many rows, for Q4_K / Q6_K / Q8_0 with K a multiple of
- * 512 and N a multiple of 256 (the engine's prefill projections), the
- * product runs on the matrix cores with fp16 operands (A and the decoded
+ * count (ds3_hip_set_dense_mfma_min_rows, default 64), and for shapes the fp16
+ * path does not take, every product is of fp32 operands, the weights decoded
+ * exactly, and summed in fp32: by VALU FMAs or, from two or three rows and for
+ * long one-row products, on the fp32 matrix cores.  The order of the sums
+ * differs between the two and from the reference kernel's (relative L2 error
+ * 1.2e-7 either way).  From that many rows, for Q4_K / Q6_K / Q8_0 with K a
+ * multiple of 512 and N a multiple of 256 (the engine's prefill projections),
+ * the product runs on the matrix cores with fp16 operands (A and the decoded
  * weights rounded to fp16, fp32 accumulation), the precision of the MoE
  * grouped products: relative L2 error ~5e-4 against fp32. */
 int ds3_hip_matmul_quantized_batch(const ds3_hip_buffer_t *A, const ds3_hip_buffer_t *W, ds3_hip_buffer_t *C,

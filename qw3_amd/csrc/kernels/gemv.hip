@@ -3,9 +3,9 @@
 // The general-purpose kernel behind the reference's vec_matmul_* and
 // matmul_quantized_batch entry points (src/ds3_metal.h:90-161).  Lanes split K
 // in 32-weight units; a group of G lanes owns one row and decodes each unit
-// once for a tile of up to 8 tokens staged in LDS.  It serves one token with
-// few or short rows, F32 rows, and rows that are no multiple of 256; the other
-// quantised products run on k_gemm32.
+// once for a tile of up to 8 tokens staged in LDS.  It serves F32 rows, rows that
+// are no multiple of 256, and the one- and two-token products that gemm32_ok
+// leaves to it; the other quantised products run on k_gemm32.
 //
 // One token over long matrices (the output head, 151,936 x 2048, and the
 // decode projections, src/ds3_engine.c:181-247) goes to k_gemv1 instead: the
@@ -183,9 +183,11 @@ static hipError_t launch_gemv1(int type, const float *x, const uint8_t *w, float
 // Measured (MI355X, us per call enqueued back to back, k_gemv before): 27 x
 // 2048 -> 768 in Q4_K 73.4 -> 7.6, Q6_K 46.0 -> 8.7, Q8_0 128 -> 8.6; 63 x 2048
 // -> 4096 480 / 259 / 920 -> 22 / 22 / 34; 40 x 4096 -> 8192 1215 / 657 / 2341
-// -> 64 / 66 / 93 (33 TFLOP/s).  Small products are bound by the launch and
-// one memory latency, large ones by the fp32 MFMA rate (33 cycles per
-// 16x16x4).
+// -> 64 / 66 / 93 (42 / 41 / 29 TFLOP/s; 40 rows take a tile of 64).  Small
+// products are bound by the launch and one or two memory latencies.  Large
+// ones are bound by the return path of the vector memory, busy 80-85 % of the
+// cycles (matrix units 30-44 %): each wave loads its A fragments itself, 64
+// pieces of 16 bytes per load, and nothing is loaded ahead of its step.
 // ---------------------------------------------------------------------------
 typedef float g32_f4 __attribute__((ext_vector_type(4)));
 typedef float g32_f4u __attribute__((ext_vector_type(4), aligned(4)));   // rows of A start on any float

@@ -842,10 +842,12 @@ k_grouped_down(const _Float16 *__restrict__ h16, int F, ExpertWeights ew, int N,
 // sets of 128 rows of W (sets N / NB apart) on gate_up's K loop; its tile comes
 // from the block index, so no list launch precedes it.  `inner` consecutive
 // tiles, on one XCD, share their W sets or, with a_first, their rows of A
-// (dense_mfma_a_first).  Bound by the weight decode, repeated for every 64 rows
-// of A: 512 x 2048 -> 4096 in Q4_K 31.3 -> 21.8 us with the conversion of A
-// (393 TFLOP/s; before, 256-row tiles from a one-workgroup list kernel left
-// half the CUs idle).
+// (dense_mfma_a_first).  Bound by no one unit: the weight decode, repeated for
+// every 64 rows of A, keeps the VALU active half of the cycles, the matrix
+// units are busy 22 %, and the two waves of a SIMD wait 37 % of theirs at chunk
+// barriers and for loads.  512 x 2048 -> 4096 in Q4_K 31.3 -> 21.8 us with the
+// conversion of A (393 TFLOP/s; before, 256-row tiles from a one-workgroup list
+// kernel left half the CUs idle).
 template <int TYPE, int NB>
 __global__ void __launch_bounds__(64 * GG_WV)
 k_dense(const _Float16 *__restrict__ x16, int K, const uint8_t *__restrict__ w, uint64_t stride, int M, int N,
